@@ -22,12 +22,14 @@
 // below it to the sums -- the next (s, t) without a second barrier. When the predicted bracket would hold more than
 // ~1500 candidates (large moves), a histogram pass over a window of twice its range goes first (2048 bins of a
 // power-of-two width, LDS histogram per block, merged by atomics), and the stage runs on the bin that holds the
-// k-th; a bracket that misses is followed by such a window on the side that holds the k-th, and round 1 takes a
-// window over 16 octaves around round 0's threshold. Round 0 (no threshold yet), and a window that misses, run
-// radix passes over the whole key range (bins of 2^21 keys, then 2^10 within the first bin, then single keys, each
+// k-th; a bracket that misses is followed by such a window on the side that holds the k-th; round 0 (no threshold yet)
+// takes a window over residuals 2^-15 .. 2, and round 1, where the first trim may have dropped the threshold by octaves, a
+// window over 16 octaves around round 0's threshold. A window that misses is followed by radix passes over the whole key range (bins of 2^21 keys, then 2^10 within the first bin, then single keys, each
 // only while the bin holds more than 2048 keys); when one key value holds the k-th and more than kCandCap
 // elements, it is the threshold and the sums take one more barrier.
 // The stage checks that its bracket holds the k-th, so a prediction can cost time but never change a result.
+// Once the moves are small, the remaining rounds need no device-wide barrier at all: each block runs them by itself on the
+// few elements whose side of the threshold may still change (run_local, in fit_k).
 //
 // Fixed point: once a round reproduces the previous round's (s, t) bit for bit, every later round would repeat
 // it exactly, so the loop stops there with the bit-identical result (on the synthetic scenes after 3 rounds).
@@ -58,7 +60,10 @@ constexpr int kFitHistSlots = 6;                       // histogram passes a rou
 constexpr int kCandCap = 32768;                        // candidates every block holds in LDS (128 KiB)
 constexpr unsigned kStageMax = 2048;                   // a pass bin with more elements is split by another pass
 constexpr double kBracketMax = 1536.0;                 // expected candidates above which a window pass goes first
-constexpr uint32_t kInvalid = 0xffffffffu;             // residual key of a padding slot: above every residual
+constexpr uint32_t kInvalid = 0xffffffffu;             // residual key of a padding slot (-1: every other key is >= 0)
+constexpr int kLocalPer = 32;                          // elements per thread of a local round, in registers
+constexpr float kLocalLow = 900.0f;                    // ... and the number below which fewer gain nothing
+constexpr unsigned kLocalCap = (unsigned)(kFitThreads * kLocalPer);
 constexpr int kFitTraceRounds = 64;
 constexpr size_t kFitHeader = 4096;                    // barrier, error flag, trace, completion count
 constexpr size_t kFitErrOffset = 64;                   // the launch's error flag
@@ -222,6 +227,7 @@ struct FitShared {
     double red[5][kFitWaves];
     unsigned tmp[kFitWaves];
     uint2 tmp2[kFitWaves];
+    alignas(16) unsigned cnt[2][2][kFitWaves];  // a local round's counts, alternating
     float s, t;
     long long kk;
     int ok;
@@ -273,6 +279,101 @@ __device__ inline void find_bin(FitShared& sh, unsigned rank, Load load, LoadBas
     __syncthreads();
 }
 
+// A box of trim-round states around (s, t, thr): |s' - s| <= Ds, |u' - u| <= Du with u = s zc + t (the line's value at
+// the mean z, which moves far less than t does), |thr' - thr| <= Dt.
+struct FitBox {
+    float s, t, thr, zc, Ds, Du, Dt;
+};
+// Whether an element's residual is below the threshold in every state of the box (`below` all ones), or above it
+// (`above` all ones), or may be either (both 0; also for NaN). |s' z + t' - tg| moves by at most Ds |z - zc| + Du, the
+// threshold by Dt; the residual's fp32 evaluation, here and in every later round, is off by at most
+// 2^-24 (3 |s z| + 2 |t| + |tg|) before the division and 2^-24 relative after it, and 2e-6 of the magnitudes covers both
+// evaluations four times over. The two tests are sign bits, not conditions: a condition combined with another goes
+// through the scalar unit, and each such hop stalls a lone wave for ~25 cycles (measured: a ballot and its count 28
+// cycles, a vector operation 5), which made these per-element loops three times longer.
+__device__ inline void fit_class(const FitBox& q, float z, float tg, int& below, int& above) {
+    const float sz = q.s * z;
+    const float e = (sz + q.t) - tg;
+    const float dm = __builtin_fmaxf(tg, 1e-3f);
+    const float m = q.Ds * __builtin_fabsf(z - q.zc) + q.Du + q.Dt * dm +
+                    (2e-6f * (__builtin_fabsf(sz) + __builtin_fabsf(q.t) + __builtin_fabsf(tg)) + 1e-30f);
+    const float x = __builtin_fabsf(e) - q.thr * dm;
+    below = (int)f2u(__builtin_fminf(x + m, 1e30f)) >> 31;  // (the minimum of a NaN and 1e30 is 1e30)
+    above = (int)f2u(__builtin_fminf(m - x, 1e30f)) >> 31;
+}
+// A condition as a word (-1 or 0) that the compiler keeps in a vector register.
+__device__ inline int word(bool c) {
+    int m = c ? -1 : 0;
+    asm("" : "+v"(m));
+    return m;
+}
+__device__ inline float masked(float x, int mask) { return u2f(f2u(x) & (uint32_t)mask); }
+
+// RN(1 / d) for the residuals' division, d >= 1e-3: the hardware reciprocal (1 ulp) and two Newton steps. Not exact for a
+// significand of all ones (and for d so large that 1 / d is denormal): fit_keys divides there.
+__device__ inline float fit_rcp(float d) {
+    float y = __builtin_amdgcn_rcpf(d);
+    y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+    return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+}
+// The keys of N elements: |((s z) + t) - tg| / max(tg, 1e-3) as ordered bits, the one operation order of every round. The
+// quotient e / d is formed from y = RN(1 / d), kept per element: q0 = e y is within 2 ulp, one correction by the exact
+// remainder makes it faithful, and a second gives the correctly rounded quotient (Markstein's theorem: y correctly
+// rounded, q faithful, r = e - q d by fused multiply-add, then RN(q + r y) = RN(e / d)). The compiler's own division
+// sequence is bit-identical, but passes a scale flag through VCC, so the N divisions ran one after the other: 16 elements
+// took 1.9 us of a round, 1.5 us this way with their masks. Operands outside the theorem's range (under- or overflow, all-ones divisors)
+// take the plain division, one branch for all N.
+template <int N>
+__device__ inline void fit_keys(float s, float t, const float* z, const float* tg, const float* rc, bool odd_targets,
+                                uint32_t* key) {
+    uint32_t emin = 0xffffffffu, emax = 0u;  // of e's bits - 1 (0 stands aside), of e's bits
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        float e = s * z[j];
+        e = e + t;
+        e = __builtin_fabsf(e - tg[j]);
+        const float d = fmax_(tg[j], 1e-3f), y = rc[j];
+        float q = e * y;
+        q = __builtin_fmaf(__builtin_fmaf(-q, d, e), y, q);
+        q = __builtin_fmaf(__builtin_fmaf(-q, d, e), y, q);
+        key[j] = f2u(q);
+        const uint32_t eb = f2u(e);
+        emin = eb - 1u < emin ? eb - 1u : emin;
+        emax = eb > emax ? eb : emax;
+    }
+    if (__any(odd_targets || emin < f2u(0x1p-60f) || emax > f2u(0x1p60f))) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            float e = s * z[j];
+            e = e + t;
+            e = e - tg[j];
+            key[j] = f2u(__builtin_fabsf(e) / fmax_(tg[j], 1e-3f));
+        }
+    }
+}
+// A target whose reciprocal fit_rcp may not round correctly, or whose quotients may leave the theorem's range.
+__device__ inline bool fit_odd_target(float tg) {
+    const float d = fmax_(tg, 1e-3f);
+    return !(d < 0x1p60f) || (~f2u(d) & 0x7fffffu) == 0u;
+}
+
+__device__ inline uint32_t wave_max_u32(uint32_t v) {
+    uint32_t o;
+    o = dpp_u32<0x111, 0xf>(v);
+    v = o > v ? o : v;
+    o = dpp_u32<0x112, 0xf>(v);
+    v = o > v ? o : v;
+    o = dpp_u32<0x114, 0xf>(v);
+    v = o > v ? o : v;
+    o = dpp_u32<0x118, 0xf>(v);
+    v = o > v ? o : v;
+    o = dpp_u32<0x142, 0xa>(v);
+    v = o > v ? o : v;
+    o = dpp_u32<0x143, 0xc>(v);
+    v = o > v ? o : v;
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 template <int kFitEPT>
 __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
     constexpr int kFitPerBlock = kFitThreads * kFitEPT;
@@ -315,7 +416,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                 mk[j] = a.mask[o0 + i];
             }
 #pragma unroll
-            for (int j = 0; j < kFitEPT; ++j) mbits |= ((vbits >> j) & (mk[j] != 0 ? 1u : 0u)) << j;
+            for (int j = 0; j < kFitEPT; ++j) mbits |= (uint32_t)word(mk[j] != 0) & vbits & (1u << j);
         } else if (a.mode == 2) {
             // the final fit on a LiDAR map of the depth map's own size (v3.py:768-775): every area window is one
             // pixel, so the pooled depth is exp(logz) itself (0 + z and z / 1 / 1 are exact) and the mask is
@@ -335,8 +436,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
 #pragma unroll
             for (int j = 0; j < kFitEPT; ++j) {
                 zr[j] = exp_f32(zr[j]);
-                const bool m = ((vbits >> j) & 1u) && lc[j] >= 2.0f && tr[j] > 0.0f && zr[j] > 0.0f && mb[j] != 0;
-                mbits |= (m ? 1u : 0u) << j;
+                mbits |= (uint32_t)(word(lc[j] >= 2.0f) & word(tr[j] > 0.0f) & word(zr[j] > 0.0f) & word(mb[j] != 0)) &
+                         vbits & (1u << j);
             }
         } else {
             // v3.py:373-378: z = exp(logz); nearest LiDAR sample (F.interpolate's index rule); mask = valid & c >= 0.999
@@ -360,19 +461,25 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             }
 #pragma unroll
             for (int j = 0; j < kFitEPT; ++j) {
-                const float d = tr[j];
-                const float c = fmin_(fmax_(lc[j] / 2.0f, 0.0f), 1.0f);
+                // finite and positive: bits in [1, 0x7f7fffff]; clamp(conf / 2, 0, 1) >= 0.999: conf / 2 >= 0.999
                 zr[j] = exp_f32(zr[j]);
-                const bool m = ((vbits >> j) & 1u) && __builtin_isfinite(d) && d > 0.0f && c >= 0.999f;
-                mbits |= (m ? 1u : 0u) << j;
+                mbits |= (uint32_t)(word(f2u(tr[j]) - 1u < 0x7f7fffffu) & word(lc[j] * 0.5f >= 0.999f)) & vbits & (1u << j);
             }
         }
 #pragma unroll
         for (int j = 0; j < kFitEPT; ++j) {  // padding slots hold zeros
-            zr[j] = ((vbits >> j) & 1u) ? zr[j] : 0.0f;
-            tr[j] = ((vbits >> j) & 1u) ? tr[j] : 0.0f;
+            const int v = (int)(vbits << (31 - j)) >> 31;
+            zr[j] = masked(zr[j], v);
+            tr[j] = masked(tr[j], v);
         }
     }
+    float ir[kFitEPT];  // 1 / max(target, 1e-3)
+#pragma unroll
+    for (int j = 0; j < kFitEPT; ++j) ir[j] = fit_rcp(fmax_(tr[j], 1e-3f));
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < kFitEPT; ++j) odd = odd || fit_odd_target(tr[j]);
+    const int npad = kFitEPT - __popc(vbits);  // padding slots: their key is negative, so the loops count them below
 
     int stage = 0;  // publish buffers alternate between consecutive publishes
     // Publishes this block's fp64 sums into buffer `stage & 1` (a bracket stage's counts ride on its barrier).
@@ -408,6 +515,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         }
     };
     float s = 1.0f, t = 0.0f;
+    float s_last = 1.0f, t_last = 0.0f;  // (s, t) before the last solve
     bool same = false;  // the last solve reproduced the previous (s, t) bit for bit
     // Closed-form weighted LS on the global sums (prompt_stem.py:222-232). The first solve: thread 0 also decides
     // the fallback and k, all threads read. Later solves: every thread holds the same sums (fixed-order block
@@ -430,6 +538,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             float ns, nt;
             ls(g, sh.ok != 0, ns, nt);
             same = f2u(ns) == f2u(s) && f2u(nt) == f2u(t);
+            s_last = s;
+            t_last = t;
             s = ns;
             t = nt;
             return;
@@ -458,19 +568,19 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
     };
 
     // ---- round 0 weights: the mask
+    float zc = 0.0f, zsd = 0.0f, itg = 0.0f;  // mean z, its standard deviation, 1 / mean target (local rounds' plan)
     {
         double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int j = 0; j < kFitEPT; ++j) {
-            if ((mbits >> j) & 1u) {
-                const double zd = zr[j], td = tr[j];
-                v[0] += 1.0;
-                v[1] += zd;
-                v[2] += td;
-                v[3] += zd * zd;
-                v[4] += zd * td;
-            }
+            const int m = (int)(mbits << (31 - j)) >> 31;
+            const double zd = masked(zr[j], m), td = masked(tr[j], m);
+            v[1] += zd;
+            v[2] += td;
+            v[3] = __builtin_fma(zd, zd, v[3]);
+            v[4] = __builtin_fma(zd, td, v[4]);
         }
+        v[0] = (double)__popc(mbits);
         FIT_MARK0(0);
         publish(v);
         FIT_MARK0(1);
@@ -479,6 +589,10 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         double g[5];
         gather_partials(g);
         ++stage;
+        const float rn = 1.0f / fmax_((float)g[0], 1.0f);
+        zc = (float)g[1] * rn;
+        zsd = __builtin_sqrtf(fmax_((float)g[3] * rn - zc * zc, 0.0f));
+        itg = (float)g[0] / fmax_((float)g[2], 1e-30f);
         solve(g, true);
     }
 
@@ -491,70 +605,573 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
     __syncthreads();
     uint32_t thr = 0, thr_prev = 0;
     bool have_prev = false;
-    // the next round's plan (see its computation at the end of a round): mode, bracket, window
-    int plan_mode = 2, plan_wsh = 0;
-    uint32_t lo = 0, hi = 0, plan_wlo = 0;
+    // the next round's plan (see its computation at the end of a round): mode, bracket, window. Round 0 has no
+    // threshold to start from: a window over relative residuals 2^-15 .. 2 in bins of 1/128 octave, one pass where
+    // the radix passes take two (round 0 at 480x640: 22.4 -> 17 us); a threshold outside it takes the radix passes.
+    int plan_mode = 1, plan_wsh = 16;
+    uint32_t lo = 0, hi = 0, plan_wlo = (127u - 15u) << 23;
+    if (a.plan_debug == 2) {
+        plan_wlo = 0x7f800001u;
+        plan_wsh = 0;
+    }
     float dens = 0.0f;  // candidates per key near the threshold, from the last stage with enough of them
+    // local rounds: the last moves of (s, u, thr) and their decayed magnitudes, elements per unit of residual near the
+    // threshold, and how often a plan of theirs has failed
+    float ds = 0.0f, du = 0.0f, dt = 0.0f, mv_s = 0.0f, mv_u = 0.0f, mv_t = 0.0f, dens_r = 0.0f;
+    int local_fails = (a.plan_debug == 2 || a.plan_debug == 3) ? 2 : 0;
+    FitBox box{};
+    // A mean displacement of the residuals over a box, relative to the target: what the number of uncertain elements is
+    // proportional to.
+    auto box_width = [&](float Ds, float Du, float Dt) { return 1.2f * (Ds * zsd + Du) * itg + Dt; };
+    // Notes the moves of the round that gave the current (s, t) and thr.
+    auto note_moves = [&](bool have) {
+        const float fthr = u2f(thr);
+        ds = s - s_last;
+        du = ds * zc + (t - t_last);
+        dt = have ? fthr - u2f(thr_prev) : 0.0f;
+        mv_s = fmax_(__builtin_fabsf(ds), 0.5f * mv_s);
+        mv_u = fmax_(__builtin_fabsf(du), 0.5f * mv_u);
+        mv_t = fmax_(fmax_(__builtin_fabsf(dt), 0.5f * mv_t), 1e-4f * fthr);
+    };
+    // The box for the rounds ahead. The moves keep their direction while they are large and shrink to a jitter, so the
+    // box reaches 0.8 c times the last move along it, and 0.3 c times the decayed magnitudes to either side; the first
+    // trim moves the threshold by -0.6 to +1.3 % (seen), mostly under 0.5: +-0.8 % after round 0. c as large as
+    // `target` uncertain elements allow, in [cmin, cmax] (above cmax while they are under kLocalLow: a wide box costs nothing
+    // there); false if that is not to be had (or nothing finite can be said).
+    auto plan_box = [&](bool have, float target, float cmin, float cmax) -> bool {
+        const float fthr = u2f(thr);
+        const float ws1 = 0.4f * __builtin_fabsf(ds) + 0.3f * mv_s, wu1 = 0.4f * __builtin_fabsf(du) + 0.3f * mv_u;
+        const float wt1 = have ? 0.4f * __builtin_fabsf(dt) + 0.8f * mv_t : 0.0f, wt0 = have ? 0.0f : 8e-3f * fthr;
+        const float u1 = 2.0f * box_width(ws1, wu1, wt1) * dens_r;
+        float c = (target - 2.0f * wt0 * dens_r) * __builtin_amdgcn_rcpf(fmax_(u1, 1e-20f));
+        const float cl = fmax_(cmax, kLocalLow * __builtin_amdgcn_rcpf(fmax_(u1, 1e-20f)));
+        c = c < cl ? c : cl;
+        if (!(c >= cmin && u1 < 1e30f && fthr < 1e12f && dens_r > 0.0f && __builtin_fabsf(s) < 1e12f &&
+              __builtin_fabsf(t) < 1e12f))
+            return false;
+        box.s = s + 0.4f * c * ds;
+        box.t = (s * zc + t + 0.4f * c * du) - box.s * zc;
+        box.thr = have ? fthr + 0.4f * c * dt : fthr;
+        box.zc = zc;
+        box.Ds = c * ws1 + 1e-6f * __builtin_fabsf(s);
+        box.Du = c * wu1 + 1e-6f * (__builtin_fabsf(s * zc) + __builtin_fabsf(t));
+        box.Dt = c * wt1 + wt0;
+        return true;
+    };
+    bool use_local = false;  // the next round runs locally (box); the plan above is then its fallback
+    auto plan_next = [&]() {
+        // ---- the next round's plan. The threshold's move from round to round (in keys, which order like the
+        // values) shrinks by 2-5x per round on the refined maps, keeps its sign while it is large, and jitters by
+        // ~10^3 keys near the fixed point. The bracket reaches a quarter of the last move against it and half a move
+        // along it, plus a margin of at least 2048 keys and ~32 expected candidates; when that bracket would hold
+        // more than kBracketMax candidates at the density the stages saw (candidates per key, kept from the last
+        // stage with at least 64), a window pass over twice that range goes first, its bins sized for 2048 over the
+        // range. A move of more than an octave is the first trim dropping the outliers of an exact point map: the
+        // next round usually repeats the threshold, so the bracket is ~256 expected candidates around it.
+        // (heuristics only, in fp32 with the hardware reciprocal: the plan never changes a result)
+        if (sh.total_cand >= 64u || dens <= 0.0f)
+            dens = (float)sh.total_cand * __builtin_amdgcn_rcpf((float)(sh.bhi_last - sh.blo_last) + 1.0f);
+        plan_mode = 2;
+        if (!have_prev && sh.total_cand >= 64u && dens * 0.016f * (float)((thr & 0x7fffffu) | 0x800000u) < 4000.0f &&
+            box_width(mv_s, mv_u, 0.0f) < 0.25f * u2f(thr)) {
+            // after round 0 of a noisy map (the first trim moved the residuals by less than a quarter of the threshold):
+            // a bracket of +-0.8 % usually holds the threshold (13 us at 480x640 against 20 by the window); the window below
+            // on a miss
+            plan_mode = 0;
+            lo = f2u(0.992f * u2f(thr));
+            hi = f2u(1.008f * u2f(thr));
+            plan_wsh = 16;
+        } else if (!have_prev) {
+            // after round 0: the first trim drops the outliers' pull, and the threshold falls by up to ~11 octaves
+            // (exact point maps) or moves by under one (noisy ones); a window from 14 octaves below to 2 above it
+            // in 2048 bins of 2^16 keys (1/128 octave) holds it
+            plan_mode = 1;
+            plan_wsh = 16;
+            plan_wlo = thr > (14u << 23) ? thr - (14u << 23) : 0u;
+        } else {
+            // keys are below 2^31 (non-negative floats, NaN included), so every range here fits 32 bits
+            const bool up = thr >= thr_prev;
+            const uint32_t am = up ? thr - thr_prev : thr_prev - thr;
+            const float rdens = dens > 0.0f ? __builtin_amdgcn_rcpf(dens) : 0.0f;
+            auto keys_for = [&](float cands) {  // keys that hold about `cands` candidates, in [2048, 2^18]
+                const float k = dens > 0.0f ? cands * rdens : 2048.0f;
+                return (uint32_t)(k < 2048.0f ? 2048.0f : (k > 262144.0f ? 262144.0f : k));
+            };
+            const bool jump = am > (1u << 23);  // a jump of over an octave predicts no move
+            uint32_t along = am / 2 + keys_for(32.0f), against = am / 4 + keys_for(32.0f);
+            if (jump) along = against = keys_for(128.0f);
+            const float expect = dens * ((float)(along + against) + 1.0f);
+            const uint32_t dn = up ? against : along, dp = up ? along : against;
+            if (expect <= kBracketMax || jump) {
+                plan_mode = 0;
+                lo = thr > dn ? thr - dn : 0u;
+                hi = thr + dp < thr ? 0xffffffffu : thr + dp;
+            } else {
+                plan_mode = 1;
+            }
+            // window bins: the smallest power of two that spans twice the bracket's range in 2048 bins
+            const uint32_t span = 2 * (along + against);
+            const int lg = 32 - __builtin_clz(span - 1u);  // ceil(log2(span)), span >= 2^13
+            plan_wsh = lg > 11 ? (lg - 11 < 21 ? lg - 11 : 21) : 0;
+            plan_wlo = thr > 2 * dn ? thr - 2 * dn : 0u;
+        }
+        // ---- the rounds ahead run locally where a box of 1.2 to 2.5 times the last moves holds at most 7000 uncertain
+        // elements at the density the stages saw (the stage and its first round then take 20 us at 480x640, 9 more than a
+        // bracket round, and every later round 5 less); not where two such plans have failed within a round each
+        use_local = false;
+        if (local_fails < 2) {
+            const float fthr = u2f(thr), h = fthr * 9.765625e-4f;
+            dens_r = dens * (float)(f2u(fthr + h) - thr) * __builtin_amdgcn_rcpf(h);
+            use_local = plan_box(have_prev, 7000.0f, 1.2f, 2.5f);
+            if (a.plan_debug == 1) {
+                box.Ds *= 0.015625f;
+                box.Du *= 0.015625f;
+            }
+        }
+        // Test hook: plans that are wrong on purpose, to exercise the fallbacks (the results must not change).
+        // 1: local rounds' boxes of a 64th of the moves (the next state leaves them), and a bracket just above its predicted range (the k-th usually lies below: a window on that side follows);
+        // 2: every plan a window above +inf (it misses: the radix passes follow); 3: windows of 2^21-key bins from
+        // 2^24 keys below the threshold (split passes with a counted below-window part).
+        if (a.plan_debug == 1 && plan_mode == 0) {
+            const uint32_t w = hi - lo;
+            lo = hi < 0xffffffffu ? hi + 1u : hi;
+            hi = lo + w < lo ? 0xffffffffu : lo + w;
+        } else if (a.plan_debug == 2) {
+            plan_mode = 1;
+            plan_wlo = 0x7f800001u;
+            plan_wsh = 0;
+        } else if (a.plan_debug == 3 && plan_mode == 1) {
+            plan_wlo = thr > (1u << 24) ? thr - (1u << 24) : 0u;
+            plan_wsh = 21;
+        }
+        thr_prev = thr;
+        have_prev = true;
+    };
+
+    // Local rounds. From the second round on (s, t) and the threshold move little, so nearly every element keeps its
+    // side of the threshold for all rounds to come. One stage classifies the elements over a box of states around the
+    // current one (plan_box) and publishes the sums over those that stay below and the uncertain rest (z, target); after
+    // its barrier every block holds the uncertain elements in its registers, and runs the remaining rounds by itself,
+    // with no further grid barrier: exact residuals and the exact k-th among the uncertain ones, their sums added to the
+    // published ones. Each round is checked: the k-th must lie in the box's threshold range (then it is the k-th of all
+    // elements), and the new (s, t) in its (s, u) range before the next round may use the classification; a round that
+    // leaves the box goes back to the grid's stages with the exact state of the rounds done. As the moves shrink the box
+    // is narrowed once it pays, and elements that become certain are folded into the sums. Every block computes the
+    // same. What bounds a local round is its chain of dependent steps in one block: residuals, two to four counting steps of one
+    // block barrier each (0.45 us), sums, the solve: 4-5 us at 1000 elements, 7 at 6000, against a bracket round's 11 at
+    // 75 blocks and 15 at 124 (publish, barrier, candidate loads). A fit of ten rounds on noisy maps, before and after:
+    // 192x256 122 -> 74 us, 240x320 122 -> 89, 480x640 141 -> 98..121, 756x1008 206 -> 138..152.
+    // Runs rounds it0, it0 + 1, ... and returns how many were completed.
+    auto run_local = [&](const int it0) -> int {
+        const unsigned kk = (unsigned)sh.kk;
+        const int lane = tid & 63, wv = tid >> 6;
+        int done = 0;
+        asm volatile("" : "+v"(mbits));
+        // ---- the stage: classify, publish, barrier
+        double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        uint32_t unc = 0;
+        int nm = 0;
+#pragma unroll
+        for (int j = 0; j < kFitEPT; ++j) {
+            int below, above;
+            fit_class(box, zr[j], tr[j], below, above);
+            const int m = (int)(mbits << (31 - j)) >> 31, inc = below & m;
+            unc |= (uint32_t)(m & ~below & ~above) & (1u << j);
+            nm -= inc;
+            const double zd = masked(zr[j], inc), td = masked(tr[j], inc);
+            v[1] += zd;
+            v[2] += td;
+            v[3] = __builtin_fma(zd, zd, v[3]);
+            v[4] = __builtin_fma(zd, td, v[4]);
+        }
+        v[0] = (double)nm;
+        unsigned nub;
+        unsigned slot = block_excl_scan((unsigned)__popc(unc), sh.tmp, nub);
+        // the pairs (z, target) take the memory of a stage's c_z and c_t together: one 8-byte load per element
+        float2* const pairs = (float2*)ws.c_z + (size_t)(stage & 1) * cap_words;
+        {
+            const size_t base = (size_t)b * kFitPerBlock;
+#pragma unroll
+            for (int g = 0; g < kFitEPT; g += 4) {
+                if (__any((unc >> g) & 15u)) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        if ((unc >> j) & 1u) {
+                            pairs[base + slot] = make_float2(zr[j], tr[j]);
+                            ++slot;
+                        }
+                    }
+                }
+            }
+        }
+        publish(v);
+        const unsigned count = fit_barrier(ws, nb, ++sync_seq, a.spin_limit, nub);
+        load_partials();
+        unsigned cc = 0;
+        if (tid < nb) cc = count < (unsigned)kFitPerBlock ? count : (unsigned)kFitPerBlock;  // (an expired wait's)
+        unsigned u;
+        const unsigned offc = block_excl_scan(cc, sh.tmp, u);
+        if (tid < nb) sh.off[tid] = offc;
+        if (tid == 0) sh.off[nb] = u;
+        __syncthreads();
+        ++stage;
+        u = (unsigned)__builtin_amdgcn_readfirstlane((int)u);
+        if (u > kLocalCap) return 0;
+        // ---- the uncertain elements into LDS in block order (thread (r, j) = (tid % nb, tid / nb) takes pairs of
+        // elements j, j + per, ... of block r's region, 16 bytes a load), then 32 to a thread
+        float2* const lds = (float2*)sh.cand;
+        static_assert(kLocalCap * 2 <= (unsigned)kCandCap, "the elements share the candidates' LDS");
+        {
+            constexpr int kHold = 16;
+            const int per = kFitThreads / nb, rr = tid % nb, jj = tid / nb;
+            const unsigned cr = jj < per ? sh.off[rr + 1] - sh.off[rr] : 0u;
+            const unsigned obase = jj < per ? sh.off[rr] : 0u;
+            const float4* const src = (const float4*)(pairs + (size_t)rr * kFitPerBlock);
+            for (unsigned s0 = (unsigned)jj; 2 * s0 < cr; s0 += (unsigned)(kHold * per)) {
+                float4 cz[kHold];
+#pragma unroll
+                for (int q = 0; q < kHold; ++q) {
+                    const unsigned e = s0 + (unsigned)(q * per);
+                    cz[q] = 2 * e < cr ? src[e] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                }
+#pragma unroll
+                for (int q = 0; q < kHold; ++q) {
+                    const unsigned e = 2 * (s0 + (unsigned)(q * per));
+                    if (e < cr) lds[obase + e] = make_float2(cz[q].x, cz[q].y);
+                    if (e + 1 < cr) lds[obase + e + 1] = make_float2(cz[q].z, cz[q].w);
+                }
+            }
+        }
+        double base[5] = {pp[0], pp[1], pp[2], pp[3], pp[4]};
+        block_sum5(base, sh.red);  // (its barriers order the LDS stores too)
+        float ez[kLocalPer], et[kLocalPer], ei[kLocalPer];
+        bool local_odd = false;
+        auto load_elements = [&]() {
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        // past the end: an element of residual 1e18, above every box (plan_box), in no sum
+                        const unsigned f = (unsigned)(j * kFitThreads + tid);
+                        const float2 e = f < u ? lds[f] : make_float2(0.0f, -1e15f);
+                        ez[j] = e.x;
+                        et[j] = e.y;
+                        ei[j] = fit_rcp(fmax_(e.y, 1e-3f));
+                        local_odd = local_odd || fit_odd_target(e.y);
+                    }
+                }
+            }
+        };
+        load_elements();
+        double s_lo = -1e300, s_hi = 1e300, u_lo = -1e300, u_hi = 1e300;
+        uint32_t k_lo = 1u, k_hi = 0x7f7fffffu;
+        // the states the current classification holds for (1e-4 of the box is kept for the margins' own rounding)
+        auto enter_box = [&]() {
+            const double us = (double)box.s * zc + box.t;
+            const double Ds = 0.9999 * box.Ds, Du = 0.9999 * box.Du;
+            s_lo = box.s - Ds > s_lo ? box.s - Ds : s_lo;
+            s_hi = box.s + Ds < s_hi ? box.s + Ds : s_hi;
+            u_lo = us - Du > u_lo ? us - Du : u_lo;
+            u_hi = us + Du < u_hi ? us + Du : u_hi;
+            const uint32_t a0 = f2u(fmax_(box.thr - 0.9999f * box.Dt, 0.0f)), a1 = f2u(box.thr + 0.9999f * box.Dt);
+            k_lo = a0 > k_lo ? a0 : k_lo;
+            k_hi = a1 < k_hi ? a1 : k_hi;
+        };
+        int par = 0;
+        uint32_t key[kLocalPer];
+        // Elements of the block with keys up to each of four pivots: one block barrier.
+        auto counts = [&](auto& p, auto& c) {
+            constexpr int P = sizeof(p) / sizeof(p[0]);
+            unsigned n[P];
+#pragma unroll
+            for (int q = 0; q < P; ++q) n[q] = 0;
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j)
+#pragma unroll
+                        for (int q = 0; q < P; ++q) n[q] += key[j] <= p[q] ? 1u : 0u;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < P; q += 2) {
+                const unsigned both = wave_incl_scan_u32(n[q] | (n[q + 1] << 16));  // at most 2048 each
+                if (lane == 63) sh.cnt[par][q / 2][wv] = both;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < P; q += 2) {
+                const uint4 v4 = *(const uint4*)sh.cnt[par][q / 2];
+                const unsigned v = (unsigned)__builtin_amdgcn_readfirstlane((int)((v4.x + v4.y) + (v4.z + v4.w)));
+                c[q] = v & 0xffffu;
+                c[q + 1] = v >> 16;
+            }
+            par ^= 1;
+        };
+        enter_box();
+        dens_r = 0.5f * (float)u * __builtin_amdgcn_rcpf(box_width(box.Ds, box.Du, box.Dt));
+
+#pragma nounroll
+        for (;;) {
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+                    fit_keys<4>(s, t, ez + g, et + g, ei + g, local_odd, key + g);
+                }
+            }
+            // ---- the k-th key: count(<= klo) = c_lo < rank <= c_hi = count(<= khi). The first step counts the range's ends
+            // and two moves' reach around the last threshold; then four counts a step, around the rank's place among
+            // evenly spread keys (a quarter and nine tenths of their number's square root to either side), then, should
+            // that not end soon, quartering
+            const unsigned n_in = (unsigned)base[0];
+            const unsigned rank = kk - n_in;
+            uint32_t klo = k_lo - 1u, khi = k_hi;
+            unsigned c_lo, c_hi;
+            if (khi <= klo || khi - klo < 4u) return done;
+            {
+                const float fthr = u2f(thr);
+                uint32_t g0 = f2u(fmax_(fthr - 2.0f * mv_t, 0.0f)), g1 = f2u(fthr + 2.0f * mv_t);
+                g0 = g0 > klo + 1u ? g0 : klo + 1u;
+                g0 = g0 < khi - 2u ? g0 : khi - 2u;
+                g1 = g1 > g0 + 1u ? g1 : g0 + 1u;
+                g1 = g1 < khi - 1u ? g1 : khi - 1u;
+                uint32_t p[4] = {klo, g0, g1, khi};
+                unsigned c[4];
+                counts(p, c);
+                if (kk <= n_in || rank <= c[0] || rank > c[3]) return done;  // outside the box's range
+                const int q = rank <= c[1] ? 0 : (rank <= c[2] ? 1 : 2);
+                klo = q == 0 ? klo : (q == 1 ? g0 : g1);
+                c_lo = c[q];
+                khi = q == 0 ? g0 : (q == 1 ? g1 : khi);
+                c_hi = c[q + 1];
+            }
+            int step = 0;
+#pragma nounroll
+            while (khi - klo > 1u && c_hi != rank && c_lo + 1u != rank) {
+                const uint32_t w = khi - klo;
+                const float fw = (float)(w - 1u);
+                uint32_t p[4];
+                float at = 0.5f * (float)w, o0 = 0.25f * (float)w, o1 = o0;
+                if (++step <= 6) {
+                    const float n = (float)(c_hi - c_lo), per = (float)w * __builtin_amdgcn_rcpf(n);
+                    const float sd = __builtin_amdgcn_sqrtf(n);
+                    at = ((float)(rank - c_lo) - 0.5f) * per;
+                    o0 = fmax_(0.25f * sd, 0.5f) * per;
+                    o1 = fmax_(0.9f * sd, 1.5f) * per;
+                }
+                const float off[4] = {at - o1, at - o0, at + o0, at + o1};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t d = (uint32_t)fmin_(fmax_(off[q], 1.0f), fw);
+                    p[q] = klo + (uint32_t)__builtin_amdgcn_readfirstlane((int)(d < w - 1u ? d : w - 1u));
+                }
+                unsigned c[4];
+                counts(p, c);
+                // the gap of (klo, p0, .., p3, khi] that holds the rank
+#pragma unroll
+                for (int q = 3; q >= 0; --q)
+                    if (c[q] >= rank) {
+                        khi = p[q];
+                        c_hi = c[q];
+                    }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (c[q] < rank) {
+                        klo = p[q];
+                        c_lo = c[q];
+                    }
+            }
+            // the k-th is the largest key up to khi (count(<= khi) = rank, or khi = klo + 1), else the smallest above
+            // klo (the complements' largest)
+            const bool largest = c_hi == rank || khi - klo == 1u;
+            uint32_t mx = 0u;
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        // keys are below 2^31: sign bits of differences select
+                        const int up = ((int)khi - (int)key[j]) >> 31, dn = ((int)klo - (int)key[j]) >> 31;
+                        const uint32_t k = largest ? key[j] & ~(uint32_t)up : ~key[j] & (uint32_t)dn;
+                        mx = k > mx ? k : mx;
+                    }
+                }
+            }
+            mx = wave_max_u32(mx);
+            if (lane == 0) sh.cnt[par][0][wv] = mx;
+            __syncthreads();
+            {
+                const uint4 o = *(const uint4*)sh.cnt[par][0];
+                mx = o.x > o.y ? o.x : o.y;
+                mx = o.z > mx ? o.z : mx;
+                mx = o.w > mx ? o.w : mx;
+            }
+            par ^= 1;
+            const uint32_t found = (uint32_t)__builtin_amdgcn_readfirstlane((int)(largest ? mx : ~mx));
+            // ---- the sums and the next (s, t)
+            double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            int nw = 0;
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        const int inc = ((int)key[j] - (int)found - 1) >> 31;
+                        nw -= inc;
+                        const double zd = masked(ez[j], inc), td = masked(et[j], inc);
+                        w[1] += zd;
+                        w[2] += td;
+                        w[3] = __builtin_fma(zd, zd, w[3]);
+                        w[4] = __builtin_fma(zd, td, w[4]);
+                    }
+                }
+            }
+            w[0] = (double)nw;
+            block_sum5(w, sh.red);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) w[k] += base[k];
+            solve(w, false);
+            thr_prev = thr;
+            thr = found;
+            if (b == 0 && tid == 0 && it0 + done < kFitTraceRounds) {
+                ws.trace[2 * (it0 + done)] = 3u | ((unsigned)(step < 15 ? step : 15) << 4) | (u << 8);
+                ws.trace[768 + it0 + done] = thr;
+                ws.trace[2 * (it0 + done) + 1] = (uint32_t)wall_clock64();
+            }
+            ++done;
+            note_moves(true);
+            const double us = (double)s * zc + t;
+            if (same || it0 + done >= a.iters || !(s >= s_lo && s <= s_hi && us >= u_lo && us <= u_hi)) return done;
+            // ---- narrow where it drops most of more than 1600 elements and two rounds are left to gain by it
+            if (u <= 1600u || it0 + done + 2 > a.iters || !plan_box(true, fmax_(0.4f * (float)u, kLocalLow), 1.2f, 16.0f))
+                continue;
+            double c5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            uint32_t keep = 0;
+            int nin = 0;
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        int below, above;
+                        fit_class(box, ez[j], et[j], below, above);
+                        keep |= (uint32_t)(~below & ~above) & (1u << j);
+                        nin -= below;
+                        const double zd = masked(ez[j], below), td = masked(et[j], below);
+                        c5[1] += zd;
+                        c5[2] += td;
+                        c5[3] = __builtin_fma(zd, zd, c5[3]);
+                        c5[4] = __builtin_fma(zd, td, c5[4]);
+                    }
+                }
+            }
+            c5[0] = (double)nin;
+            unsigned left;
+            unsigned pos = block_excl_scan((unsigned)__popc(keep), sh.tmp, left);
+#pragma unroll
+            for (int g = 0; g < kLocalPer; g += 4) {
+                if ((unsigned)(g * kFitThreads) < u) {
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        if ((keep >> j) & 1u) {
+                            lds[pos] = make_float2(ez[j], et[j]);
+                            ++pos;
+                        }
+                    }
+                }
+            }
+            block_sum5(c5, sh.red);  // (and the stores are ordered)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) base[k] += c5[k];
+            u = (unsigned)__builtin_amdgcn_readfirstlane((int)left);
+            load_elements();
+            enter_box();
+            dens_r = 0.5f * (float)u * __builtin_amdgcn_rcpf(box_width(box.Ds, box.Du, box.Dt));
+        }
+    };
 
     // A fit that falls back to (1, 0) never changes (s, t): its trim rounds cannot affect the result.
     int rounds = 0;  // trim rounds run (the loop stops early at a fixed point)
     for (int it = 0; it < (sh.ok ? a.iters : 0); ++it) {
+        if (use_local) {
+            const int done = run_local(it);
+            it += done;
+            rounds = it;
+            if (same || it >= a.iters) break;
+            if (done < 2) ++local_fails;
+            use_local = false;
+            if (done > 0) plan_next();
+            if (use_local) {
+                --it;
+                continue;
+            }
+        }
         rounds = it + 1;
         // The element values and mask bits are loop-invariant; hiding that from the compiler keeps it from hoisting
         // their fp64 products and per-element lane masks out of the loop into hundreds of extra registers.
 #pragma unroll
-        for (int j = 0; j < kFitEPT; ++j) asm volatile("" : "+v"(zr[j]), "+v"(tr[j]));
+        for (int j = 0; j < kFitEPT; ++j) asm volatile("" : "+v"(zr[j]), "+v"(tr[j]), "+v"(ir[j]));
         asm volatile("" : "+v"(mbits), "+v"(vbits));
         // ---- relative residuals as ordered bit patterns (+inf off the mask, kInvalid on padding)
         uint32_t rb[kFitEPT];
+        fit_keys<kFitEPT>(s, t, zr, tr, ir, odd, rb);
 #pragma unroll
         for (int j = 0; j < kFitEPT; ++j) {
-            float e = s * zr[j];
-            e = e + t;
-            e = e - tr[j];
-            const float r = __builtin_fabsf(e) / fmax_(tr[j], 1e-3f);
-            const uint32_t rm = ((mbits >> j) & 1u) ? f2u(r) : 0x7f800000u;
-            rb[j] = ((vbits >> j) & 1u) ? rm : kInvalid;
+            // off the mask +inf, padding kInvalid (bit fields of mbits and vbits, no conditions)
+            const uint32_t m = (uint32_t)((int)(mbits << (31 - j)) >> 31), v = (uint32_t)((int)(vbits << (31 - j)) >> 31);
+            rb[j] = (rb[j] & m) | (0x7f800000u & ~m) | ~v;
         }
         const unsigned kk = (unsigned)sh.kk;
 
         // Publishes below-count, below-sums and the candidates in [blo, bhi]; then a barrier; then the totals.
         auto stage_bracket = [&](uint32_t blo, uint32_t bhi) {
+            blo = blo < 0x7fffffffu ? blo : 0x7fffffffu;
+            bhi = bhi < 0x7fffffffu ? bhi : 0x7fffffffu;
             FIT_MARK(0);
             asm volatile("" : "+v"(mbits), "+v"(vbits));  // no per-element lane masks kept across phases
-            // branch-free: below-count, masked below-sums (fp64; z*z and z*t are exact in fp64), candidate count
+            // branch-free: below-count, masked below-sums (fp64; z*z and z*t are exact in fp64, so the fused form rounds
+            // once, as the sum alone would), candidate count. Keys are below 2^31 (padding is -1), so comparisons are
+            // sign bits of differences
             double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            unsigned below = 0, nc = 0, nm = 0;
+            int below = -npad, nc = 0, nm = 0;
+            uint32_t cm = 0;
 #pragma unroll
             for (int j = 0; j < kFitEPT; ++j) {
-                const uint32_t k = rb[j];
-                const bool isb = k < blo;
-                const bool inc = isb && ((mbits >> j) & 1u);
-                below += isb ? 1u : 0u;
-                nm += inc ? 1u : 0u;
-                nc += (!isb && k <= bhi) ? 1u : 0u;
-                const double zd = inc ? (double)zr[j] : 0.0;
-                const double td = inc ? (double)tr[j] : 0.0;
+                const int k = (int)rb[j];
+                const int isb = (k - (int)blo) >> 31;
+                const int isc = ~isb & ~(((int)bhi - k) >> 31);
+                const int inc = isb & ((int)(mbits << (31 - j)) >> 31);
+                below -= isb;
+                nc -= isc;
+                nm -= inc;
+                cm |= (uint32_t)isc & (1u << j);
+                const double zd = masked(zr[j], inc), td = masked(tr[j], inc);
                 v[1] += zd;
                 v[2] += td;
-                v[3] += zd * zd;
-                v[4] += zd * td;
+                v[3] = __builtin_fma(zd, zd, v[3]);
+                v[4] = __builtin_fma(zd, td, v[4]);
             }
             v[0] = (double)nm;
             // one scan for both counts: below in the high half, candidates in the low half (each <= 8192 per block)
             unsigned packed_total;
-            const unsigned packed = block_excl_scan((below << 16) | nc, sh.tmp, packed_total);
+            const unsigned packed = block_excl_scan(((unsigned)below << 16) | (unsigned)nc, sh.tmp, packed_total);
             unsigned slot = packed & 0xffffu;
             const unsigned ncb = packed_total & 0xffffu;
             const size_t base = (size_t)(stage & 1) * cap_words + (size_t)b * kFitPerBlock;
 #pragma unroll
-            for (int j = 0; j < kFitEPT; ++j) {
-                const uint32_t k = rb[j];
-                if (k >= blo && k <= bhi) {
-                    ws.c_key[base + slot] = k | (((mbits >> j) & 1u) << 31);
-                    ws.c_z[base + slot] = zr[j];
-                    ws.c_t[base + slot] = tr[j];
-                    ++slot;
+            for (int g = 0; g < kFitEPT; g += 4) {
+                if (__any((cm >> g) & 15u)) {  // few elements are candidates: most waves skip most groups
+#pragma unroll
+                    for (int j = g; j < g + 4; ++j) {
+                        if ((cm >> j) & 1u) {
+                            ws.c_key[base + slot] = rb[j] | (((mbits >> j) & 1u) << 31);
+                            ws.c_z[base + slot] = zr[j];
+                            ws.c_t[base + slot] = tr[j];
+                            ++slot;
+                        }
+                    }
                 }
             }
             publish(v);
@@ -698,18 +1315,18 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             // sums: this thread's share of the published below-partials, then its candidates at or under thr in
             // flat order; then one fixed-order block reduction
             double v[5] = {pp[0], pp[1], pp[2], pp[3], pp[4]};
+            int nsel = 0;
 #pragma unroll
             for (int u = 0; u < kHold; ++u) {
-                const uint32_t w = hw[u];
-                if ((w >> 31) && (w & 0x7fffffffu) <= thr) {
-                    const double zd = hz[u], td = ht[u];
-                    v[0] += 1.0;
-                    v[1] += zd;
-                    v[2] += td;
-                    v[3] += zd * zd;
-                    v[4] += zd * td;
-                }
+                const int inc = ((int)hw[u] >> 31) & (((int)(hw[u] & 0x7fffffffu) - (int)thr - 1) >> 31);
+                const double zd = masked(hz[u], inc), td = masked(ht[u], inc);
+                nsel -= inc;
+                v[1] += zd;
+                v[2] += td;
+                v[3] = __builtin_fma(zd, zd, v[3]);
+                v[4] = __builtin_fma(zd, td, v[4]);
             }
+            v[0] += (double)nsel;
             for (unsigned s0 = (unsigned)(jj + kHold * per); s0 < cr; s0 += (unsigned)(kHold * per)) {
                 // kHold candidates per trip: all loads issued before any is used
                 float cz[kHold], ct[kHold];
@@ -729,8 +1346,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                         v[0] += 1.0;
                         v[1] += zd;
                         v[2] += td;
-                        v[3] += zd * zd;
-                        v[4] += zd * td;
+                        v[3] = __builtin_fma(zd, zd, v[3]);
+                        v[4] = __builtin_fma(zd, td, v[4]);
                     }
                 }
             }
@@ -757,15 +1374,17 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             for (int q = tid; q < kFitBins; q += kFitThreads) sh.hist[q] = 0;
             if (tid == 0) sh.hbelow = 0;
             __syncthreads();
-            unsigned nbelow = 0;
+            // one comparison per element (around its LDS atomic): the window's keys are [wlo, wlo + span), span at most
+            // 2^31; a key below wlo and a padding slot's -1 give a difference of 2^31 or more
+            const uint32_t span = wsh < 20 ? (uint32_t)kFitBins << wsh : 0x80000000u;
+            int below_n = -npad;
 #pragma unroll
-            for (int j = 0; j < kFitEPT; ++j) {  // one branch per element (around its LDS atomic)
-                const uint32_t k = rb[j];
-                const bool v = (vbits >> j) & 1u;
-                const uint32_t q = (k - wlo) >> wsh;
-                nbelow += (v && k < wlo) ? 1u : 0u;
-                if (v && k >= wlo && q < (uint32_t)kFitBins) atomicAdd(&sh.hist[q], 1u);
+            for (int j = 0; j < kFitEPT; ++j) {
+                const uint32_t d = rb[j] - wlo;
+                below_n -= ((int)rb[j] - (int)wlo) >> 31;
+                if (d < span) atomicAdd(&sh.hist[d >> wsh], 1u);
             }
+            unsigned nbelow = (unsigned)below_n;
             const bool count_below = below == kNoBelow;
             if (count_below) {
                 nbelow = wave_incl_scan_u32(nbelow);
@@ -774,8 +1393,14 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             __syncthreads();
             unsigned* gh = ws.hist + ((int64_t)it * kFitHistSlots + hslot) * kFitHistWords;
             hslot = hslot + 1 < kFitHistSlots ? hslot + 1 : hslot;  // at most 6 passes a round (never reached)
-            for (int q = tid; q < kFitBins; q += kFitThreads)
-                if (sh.hist[q]) atomicAdd(&gh[q], sh.hist[q]);
+            {
+                unsigned h[kFitBins / kFitThreads];  // all read before any is merged
+#pragma unroll
+                for (int q = 0; q < kFitBins / kFitThreads; ++q) h[q] = sh.hist[q * kFitThreads + tid];
+#pragma unroll
+                for (int q = 0; q < kFitBins / kFitThreads; ++q)
+                    if (h[q]) atomicAdd(&gh[q * kFitThreads + tid], h[q]);
+            }
             if (count_below && tid == 0 && sh.hbelow) atomicAdd(&gh[kFitBins + (b & 15)], sh.hbelow);
             fit_barrier(ws, nb, ++sync_seq, a.spin_limit);
             find_bin(
@@ -848,8 +1473,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                             v[0] += 1.0;
                             v[1] += zd;
                             v[2] += td;
-                            v[3] += zd * zd;
-                            v[4] += zd * td;
+                            v[3] = __builtin_fma(zd, zd, v[3]);
+                            v[4] = __builtin_fma(zd, td, v[4]);
                         }
                     }
                     publish(v);
@@ -881,7 +1506,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                 wlo = blo;
                 wsh = 0;
                 while (((uint64_t)kFitBins << wsh) < (uint64_t)bhi - blo + 1u && wsh < 21) ++wsh;
-            } else if (bhi == 0xffffffffu) {
+            } else if (bhi >= 0x7fffffffu) {
                 mode = 2;
                 path = 1;
             } else {
@@ -897,71 +1522,9 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         // Fixed point: when a round reproduces the previous (s, t) bit for bit, the next round sees the same
         // residuals, hence the same k-th value, weights and sums, so every remaining round -- and the final
         // solve -- returns exactly these (s, t). Stopping here gives the bit-identical result.
-        // ---- the next round's plan. The threshold's move from round to round (in keys, which order like the
-        // values) shrinks by 2-5x per round on the refined maps, keeps its sign while it is large, and jitters by
-        // ~10^3 keys near the fixed point. The bracket reaches a quarter of the last move against it and half a move
-        // along it, plus a margin of at least 2048 keys and ~32 expected candidates; when that bracket would hold
-        // more than kBracketMax candidates at the density the stages saw (candidates per key, kept from the last
-        // stage with at least 64), a window pass over twice that range goes first, its bins sized for 2048 over the
-        // range. A move of more than an octave is the first trim dropping the outliers of an exact point map: the
-        // next round usually repeats the threshold, so the bracket is ~256 expected candidates around it.
-        if (same) break;  // the fixed point below: no next round to plan
-        // (heuristics only, in fp32 with the hardware reciprocal: the plan never changes a result)
-        if (sh.total_cand >= 64u || dens <= 0.0f)
-            dens = (float)sh.total_cand * __builtin_amdgcn_rcpf((float)(sh.bhi_last - sh.blo_last) + 1.0f);
-        plan_mode = 2;
-        if (!have_prev) {
-            // after round 0: the first trim drops the outliers' pull, and the threshold falls by up to ~11 octaves
-            // (exact point maps) or moves by under one (noisy ones); a window from 14 octaves below to 2 above it
-            // in 2048 bins of 2^16 keys (1/128 octave) holds it
-            plan_mode = 1;
-            plan_wsh = 16;
-            plan_wlo = thr > (14u << 23) ? thr - (14u << 23) : 0u;
-        } else {
-            // keys are below 2^31 (non-negative floats, NaN included), so every range here fits 32 bits
-            const bool up = thr >= thr_prev;
-            const uint32_t am = up ? thr - thr_prev : thr_prev - thr;
-            const float rdens = dens > 0.0f ? __builtin_amdgcn_rcpf(dens) : 0.0f;
-            auto keys_for = [&](float cands) {  // keys that hold about `cands` candidates, in [2048, 2^18]
-                const float k = dens > 0.0f ? cands * rdens : 2048.0f;
-                return (uint32_t)(k < 2048.0f ? 2048.0f : (k > 262144.0f ? 262144.0f : k));
-            };
-            const bool jump = am > (1u << 23);  // a jump of over an octave predicts no move
-            uint32_t along = am / 2 + keys_for(32.0f), against = am / 4 + keys_for(32.0f);
-            if (jump) along = against = keys_for(128.0f);
-            const float expect = dens * ((float)(along + against) + 1.0f);
-            const uint32_t dn = up ? against : along, dp = up ? along : against;
-            if (expect <= kBracketMax || jump) {
-                plan_mode = 0;
-                lo = thr > dn ? thr - dn : 0u;
-                hi = thr + dp < thr ? 0xffffffffu : thr + dp;
-            } else {
-                plan_mode = 1;
-            }
-            // window bins: the smallest power of two that spans twice the bracket's range in 2048 bins
-            const uint32_t span = 2 * (along + against);
-            const int lg = 32 - __builtin_clz(span - 1u);  // ceil(log2(span)), span >= 2^13
-            plan_wsh = lg > 11 ? (lg - 11 < 21 ? lg - 11 : 21) : 0;
-            plan_wlo = thr > 2 * dn ? thr - 2 * dn : 0u;
-        }
-        // Test hook: plans that are wrong on purpose, to exercise the fallbacks (the results must not change).
-        // 1: a bracket just above its predicted range (the k-th usually lies below: a window on that side follows);
-        // 2: every plan a window above +inf (it misses: the radix passes follow); 3: windows of 2^21-key bins from
-        // 2^24 keys below the threshold (split passes with a counted below-window part).
-        if (a.plan_debug == 1 && plan_mode == 0) {
-            const uint32_t w = hi - lo;
-            lo = hi < 0xffffffffu ? hi + 1u : hi;
-            hi = lo + w < lo ? 0xffffffffu : lo + w;
-        } else if (a.plan_debug == 2) {
-            plan_mode = 1;
-            plan_wlo = 0x7f800001u;
-            plan_wsh = 0;
-        } else if (a.plan_debug == 3 && plan_mode == 1) {
-            plan_wlo = thr > (1u << 24) ? thr - (1u << 24) : 0u;
-            plan_wsh = 21;
-        }
-        thr_prev = thr;
-        have_prev = true;
+        if (same) break;
+        note_moves(have_prev);
+        plan_next();
     }
 
     if (b == 0 && tid == 0) {

@@ -586,7 +586,7 @@ def test_fit_expired_wait_is_reported_and_does_not_leak(gpu, libpmg):
 
 def _fit_trace(ws: "torch.Tensor"):
     """Block 0's round record in the fit workspace: per round the selection path code (low 3 bits: 0 bracket,
-    1 bracket missed -> radix, 2 radix, 4 window, 5 bracket missed -> window, 6 window missed -> radix, 7 both
+    1 bracket missed -> radix, 2 radix, 3 local, 4 window, 5 bracket missed -> window, 6 window missed -> radix, 7 both
     missed -> radix; bit 3: one-value threshold) and the histogram passes; the number of rounds run."""
     tr = ws[128:128 + 4096].cpu().numpy().view(np.uint32)
     rounds = int(tr[130])
@@ -686,6 +686,42 @@ def test_fit_random_cases_and_forced_plans(gpu, libpmg):
             assert thr0 == np.float32(info_o[0]["thr"]).view(np.int32), case
         for mode in (1, 2, 3):
             assert res[mode] == res[0], (case, mode, res[mode], res[0])
+
+
+@pytest.mark.parametrize("N", [33, 4_095, 4_097, 75 * 4_096 + 1, 1 << 19, (1 << 19) + 1, 256 * 24 * 256 + 1])
+def test_fit_local_rounds(gpu, libpmg, N):
+    """The local rounds (the uncertain elements in every block, no grid barrier) at the edges of the element layouts (one
+    block, one element into the next, 16 / 24 / 32 per thread): the thresholds and (s, t) of the grid's own rounds, which
+    plan 3 keeps to, bit for bit, and the fp64 oracle's. Noisy targets, so that all ten rounds move; a few targets
+    with an all-ones significand and of 1e-3 or less (the residuals' division by a kept reciprocal)."""
+    announce(f"fit local rounds N={N}")
+    rng = np.random.default_rng(N)
+    z = rng.uniform(0.4, 6, size=N).astype(np.float32)
+    t = (1.3 * z + 0.05 + 0.02 * z * rng.normal(size=N)).astype(np.float32)
+    t = np.where(rng.random(N) < 0.05, t * rng.uniform(0.4, 1.8, size=N), t).astype(np.float32)
+    t[::53] = np.nextafter(np.float32(2.0), np.float32(0.0))
+    t[7::97] = np.float32(5e-4)
+    m = rng.random(N) < 0.8
+    m[:33] = True
+    out, codes = [], []
+    try:
+        for mode in (0, 1, 3):
+            libpmg.pmg_debug_fit_plan(mode)
+            s_, t_, info = ops.fit_scale_shift(_t(z[None], gpu), _t(t[None], gpu), _t(m[None], gpu), iters=10, return_info=True)
+            torch.cuda.synchronize()
+            codes.append({c for c, _ in _fit_trace(ops._fit_workspace(0, s_.device))})
+            assert int(info[0, 4]) == 0
+            out.append((float(s_[0]), float(t_[0]), int(info[0, 3])))
+    finally:
+        libpmg.pmg_debug_fit_plan(0)
+    assert out[1] == out[0] and out[2] == out[0], out
+    so, to, info_o = ofit.fit_f64(z[None], t[None], m[None], iters=10, return_info=True)
+    _close_st(out[0][0], out[0][1], so[0], to[0])
+    if np.float32(out[0][0]) == so[0] and np.float32(out[0][1]) == to[0]:
+        assert out[0][2] == np.float32(info_o[0]["thr"]).view(np.int32)
+    assert 3 not in codes[2]
+    # (few elements converge before a local plan; of 1.5 million, over 7000 stay uncertain until the last rounds)
+    assert not 4_000 < N < 1_000_000 or 3 in codes[0], codes[0]
 
 
 @pytest.mark.parametrize("name", ["B", "A", "H"])
