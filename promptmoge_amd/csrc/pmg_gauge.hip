@@ -4,15 +4,21 @@
 //
 //   gauge_inputs_k  one thread per LiDAR pixel: the area-pooled valid depth z_lr (the window sums of
 //                   where(ok, depth, 0) and of ok, each / height / width, as F.interpolate(mode='area')), the mask
-//                   conf >= 2 & lidar > 0 & z_lr > 0 and y = log(max(lidar, 1e-3)) - log(max(z_lr, 1e-3))
-//   per IRLS round  gauge_sums_k (a grid of blocks per frame: fp64 partial sums of the weighted normal equations
-//                   (A w)^T (A w) c = (A w)^T (y w) over the confident pixels), gauge_solve_k (one wave per frame:
-//                   the partials in a fixed order, Gaussian elimination with partial pivoting; the reference runs
-//                   LAPACK least squares on the same fp32 products), and, for every round but the last, the exact
-//                   lower median of |y - A c| (fp32 residuals) by three radix passes over its bits (gauge_hist_k:
-//                   grid-wide 2048-bin histograms of the candidates; gauge_select_k: the bucket holding the rank)
-//                   and the weights min(2 sc / max(|r|, 1e-6), 1), sc = 1.4826 median + 1e-4 (gauge_weights_k)
-//   gauge_apply_k   one thread per output pixel: exp of the polynomial (a sequential fp32 sum over the basis)
+//                   conf >= 2 & lidar > 0 & z_lr > 0, y = log(max(lidar, 1e-3)) - log(max(z_lr, 1e-3)), and the first
+//                   round's sums: fp64 partials per block of the weighted normal equations (A w)^T (A w) c = (A w)^T (y w)
+//   per IRLS round but the last
+//     gauge_resid_k   solves the round's system (every block, from the same partials in the same order: Gaussian
+//                     elimination with partial pivoting; the reference runs LAPACK least squares on the same fp32
+//                     products), writes the fp32 residuals |y - A c| and counts them into bins of 1/128 octave
+//     gauge_pick_k    finds the bin holding the exact lower median and lists its residuals
+//     gauge_sums_k    selects the median among them, forms the weights min(2 sc / max(|r|, 1e-6), 1),
+//                     sc = 1.4826 median + 1e-4, and sums the next round's system
+//   gauge_apply_k   solves the last system; per output pixel exp of the polynomial (a sequential fp32 sum over the basis)
+//
+// What bounds it: launches and the chain of small phases in them (the data is 0.4 MB at a 192x256 LiDAR map). Every step
+// that one block or wave did for the whole frame in a launch of its own (the reduction of the partials, the solve, the
+// median's bin) is done by all blocks of the next kernel instead, from the same data in the same order: 8 launches for
+// three rounds where there were 22. Measured (depth 480x640, LiDAR 192x256, the whole call): 200 -> 55 us.
 //
 // The basis is (1, u, v) or (1, u, v, u^2, uv, v^2) on torch.linspace(-1, 1, n) grids (the scalar rule: step
 // 2 / (n - 1) in fp32, start + step i for the first half, end - step (n - 1 - i) for the second). A frame with
@@ -44,50 +50,24 @@ __device__ inline void gauge_basis(float u, float v, float (&a)[kGaugeMaxK]) {
     a[5] = v * v;
 }
 
-__global__ __launch_bounds__(256) void gauge_inputs_k(const float* __restrict__ depth, const float* __restrict__ lidar,
-                                                      const float* __restrict__ conf, int H, int W, int h, int w,
-                                                      int64_t n_out, float* __restrict__ y_out,
-                                                      uint8_t* __restrict__ m_out) {
-    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (q >= n_out) return;
-    const int64_t plane = (int64_t)h * w;
-    const int64_t b = q / plane;
-    const int rem = (int)(q - b * plane);
-    const int oh = rem / w, ow = rem - oh * w;
-    const int r0 = (int)(((int64_t)oh * H) / h), r1 = (int)((((int64_t)oh + 1) * H + h - 1) / h);
-    const int c0 = (int)(((int64_t)ow * W) / w), c1 = (int)((((int64_t)ow + 1) * W + w - 1) / w);
-    const float* db = depth + b * H * W;
-    float num = 0.0f, den = 0.0f;
-    for (int r = r0; r < r1; ++r)
-        for (int c = c0; c < c1; ++c) {
-            const float d = db[(int64_t)r * W + c];
-            const bool ok = __builtin_isfinite(d) && d > 0.0f;
-            num = num + (ok ? d : 0.0f);
-            den = den + (ok ? 1.0f : 0.0f);
-        }
-    const float kh = (float)(r1 - r0), kw = (float)(c1 - c0);
-    const float nump = num / kh / kw, denp = den / kh / kw;
-    const float z = denp > 0.5f ? nump / fmax_(denp, 1e-6f) : 0.0f;
-    const float ld = lidar[q];
-    const float cf = conf ? conf[q] : 2.0f;
-    y_out[q] = log_f32(fmax_(ld, 1e-3f)) - log_f32(fmax_(z, 1e-3f));
-    m_out[q] = (cf >= 2.0f && ld > 0.0f && z > 0.0f) ? 1 : 0;
-}
-
-// ---- the IRLS rounds, spread over the GPU: per round a grid of blocks sums the weighted normal equations
-// (fp64 partials per block), one wave per frame reduces them in a fixed order and solves; then (all but the last
-// round) three radix-select passes over the residual bits (11 + 11 + 10 bits: a grid-wide histogram of the
-// candidates, then one block per frame picks the bucket holding the median's rank) and the new weights.
-constexpr int kGaugeBlk = 256;       // threads of the grid kernels
-constexpr int kGaugeMaxBlocks = 256; // blocks per frame
+constexpr int kGaugeBlk = 256;        // threads of the grid kernels
+constexpr int kGaugeMaxBlocks = 256;  // blocks per frame
 constexpr int kGaugeBins = 2048;
-constexpr int kGaugeVals = 28;       // 21 normal-matrix entries + 6 right-hand sides + count (K = 6; fewer for 3)
+constexpr int kGaugeHist = kGaugeBins + 8;  // the bins, the count below them, padding
+constexpr int kGaugeVals = 28;        // 21 normal-matrix entries + 6 right-hand sides + count (K = 6; fewer for 3)
+constexpr int kGaugeList = 4096;      // listed residuals a block keeps in LDS
+// The bins: 16 octaves of residuals, 2^-18 .. 2^-2, in 2^16 keys (fp32 bit patterns) each. A median outside them lists
+// all residuals on its side.
+constexpr uint32_t kGaugeLow = (127u - 18u) << 23;
+constexpr int kGaugeShift = 16;
 
 struct GaugeState {
-    uint32_t prefix;  // median bits found so far
-    uint32_t rank;    // rank of the median among the candidates with that prefix
-    int32_t count;    // confident pixels
-    int32_t valid;    // 1 while the frame has a finite solution
+    int32_t valid[2];  // by the round's parity: the frame has a finite solution so far
+    uint32_t rank;     // rank of the lower median among the confident pixels' residuals
+    uint32_t listed;   // residuals listed by gauge_pick_k
+    uint32_t key_lo, key_hi;  // the listed range of keys
+    uint32_t list_rank;       // rank of the median among the listed
+    uint32_t pad;
 };
 
 __device__ inline void gauge_range(int64_t N, int nblk, int blk, int64_t& n0, int64_t& n1) {
@@ -95,279 +75,442 @@ __device__ inline void gauge_range(int64_t N, int nblk, int blk, int64_t& n0, in
     n1 = N * (blk + 1) / nblk;
 }
 
+// Adds one pixel's terms to a thread's sums: the upper triangle of (A w)^T (A w), then (A w)^T (y w) (products of
+// two floats are exact in fp64, so the fused form rounds once, as the sum alone would).
 template <int K>
-__global__ __launch_bounds__(kGaugeBlk) void gauge_sums_k(const float* __restrict__ y_all,
-                                                          const uint8_t* __restrict__ m_all,
-                                                          const float* __restrict__ w_all, int h, int w, int first,
-                                                          const GaugeState* __restrict__ st, int nblk,
-                                                          double* __restrict__ partials) {
+__device__ inline void gauge_add(const float (&a)[kGaugeMaxK], float y, float wn, double* G) {
     constexpr int NG = K * (K + 1) / 2;
+    float wa[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) wa[k] = a[k] * wn;
+    const float wy = y * wn;
+    int e = 0;
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+#pragma unroll
+        for (int j = i; j < K; ++j, ++e) G[e] = __builtin_fma((double)wa[i], (double)wa[j], G[e]);
+#pragma unroll
+    for (int i = 0; i < K; ++i) G[NG + i] = __builtin_fma((double)wa[i], (double)wy, G[NG + i]);
+    G[NG + K] += 1.0;
+}
+
+// A block's sums into its partials (DPP wave scans, then the waves in order).
+template <int K>
+__device__ inline void gauge_publish(const double* G, double* partials) {
+    constexpr int NV = K * (K + 1) / 2 + K + 1;
     __shared__ double s_red[kGaugeBlk / 64][kGaugeVals];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const double v = wave_incl_scan_f64(G[k]);
+        if (lane == 63) s_red[wv][k] = v;
+    }
+    __syncthreads();
+    if (tid < NV) {
+        double v = 0.0;
+        for (int q = 0; q < kGaugeBlk / 64; ++q) v += s_red[q][tid];
+        partials[tid] = v;
+    }
+}
+
+// The frame's system from its nblk partials (eight runs of blocks, then the runs in order) and its solution, in every
+// thread of every block alike. Returns whether the frame has a solution (v3.py:174-175: at least 200 confident pixels;
+// a finite one) and the count of confident pixels.
+template <int K>
+__device__ inline bool gauge_solve(const double* partials, int nblk, float (&cf)[kGaugeMaxK], int& count) {
+    constexpr int NG = K * (K + 1) / 2, NV = NG + K + 1;
+    __shared__ double s_run[8][32];
+    __shared__ double s_v[32];
+    const int tid = threadIdx.x, val = tid & 31, run = tid >> 5;
+    double acc = 0.0;
+    if (val < NV) {
+#pragma unroll 8
+        for (int q = run; q < nblk; q += 8) acc += partials[(int64_t)q * kGaugeVals + val];
+    }
+    s_run[run][val] = acc;
+    __syncthreads();
+    if (tid < NV) {
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v += s_run[q][tid];
+        s_v[tid] = v;
+    }
+    __syncthreads();
+    count = (int)s_v[NG + K];
+    double A[K][K + 1];
+    {
+        int e = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+#pragma unroll
+            for (int j = i; j < K; ++j, ++e) A[i][j] = A[j][i] = s_v[e];
+            A[i][K] = s_v[NG + i];
+        }
+    }
+    // Gaussian elimination on [G | g], the largest pivot brought up by conditional swaps (registers, no indexing)
+    bool ok = count >= kGaugeMinPoints;
+    double inv[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+#pragma unroll
+        for (int r = c + 1; r < K; ++r) {
+            const bool swap = fabs(A[r][c]) > fabs(A[c][c]);
+#pragma unroll
+            for (int k = c; k <= K; ++k) {
+                const double x = A[c][k], y = A[r][k];
+                A[c][k] = swap ? y : x;
+                A[r][k] = swap ? x : y;
+            }
+        }
+        ok = ok && fabs(A[c][c]) > 0.0;
+        inv[c] = 1.0 / A[c][c];
+#pragma unroll
+        for (int r = c + 1; r < K; ++r) {
+            const double f = A[r][c] * inv[c];
+#pragma unroll
+            for (int k = c + 1; k <= K; ++k) A[r][k] -= f * A[c][k];
+        }
+    }
+    double x[K];
+#pragma unroll
+    for (int c = K - 1; c >= 0; --c) {
+        double v = A[c][K];
+#pragma unroll
+        for (int k = c + 1; k < K; ++k) v -= A[c][k] * x[k];
+        x[c] = v * inv[c];
+    }
+#pragma unroll
+    for (int k = 0; k < kGaugeMaxK; ++k) {
+        cf[k] = k < K ? (float)x[k < K ? k : 0] : 0.0f;
+        ok = ok && __builtin_isfinite(cf[k]);
+    }
+    return ok;
+}
+
+template <int K>
+__global__ __launch_bounds__(kGaugeBlk) void gauge_inputs_k(const float* __restrict__ depth,
+                                                            const float* __restrict__ lidar,
+                                                            const float* __restrict__ conf, int H, int W, int h, int w,
+                                                            int nblk, float* __restrict__ y_out,
+                                                            uint8_t* __restrict__ m_out, uint32_t* __restrict__ hist,
+                                                            double* __restrict__ partials) {
     const int b = blockIdx.y, tid = threadIdx.x;
-    if (!first && !st[b].valid) return;
+    const int64_t N = (int64_t)h * w, base = (int64_t)b * N;
+    for (int i = blockIdx.x * kGaugeBlk + tid; i < kGaugeHist; i += nblk * kGaugeBlk) hist[(int64_t)b * kGaugeHist + i] = 0u;
+    int64_t n0, n1;
+    gauge_range(N, nblk, blockIdx.x, n0, n1);
+    const float* db = depth + (int64_t)b * H * W;
+    double G[K * (K + 1) / 2 + K + 1] = {};
+    for (int64_t n = n0 + tid; n < n1; n += kGaugeBlk) {
+        const int oh = (int)(n / w), ow = (int)(n - (int64_t)oh * w);
+        const int r0 = (int)(((int64_t)oh * H) / h), r1 = (int)((((int64_t)oh + 1) * H + h - 1) / h);
+        const int c0 = (int)(((int64_t)ow * W) / w), c1 = (int)((((int64_t)ow + 1) * W + w - 1) / w);
+        const float ld = lidar[base + n];
+        const float cfd = conf ? conf[base + n] : 2.0f;
+        float num = 0.0f, den = 0.0f;
+        for (int r = r0; r < r1; ++r)
+            for (int c = c0; c < c1; ++c) {
+                const float d = db[(int64_t)r * W + c];
+                const bool ok = __builtin_isfinite(d) && d > 0.0f;
+                num = num + (ok ? d : 0.0f);
+                den = den + (ok ? 1.0f : 0.0f);
+            }
+        const float kh = (float)(r1 - r0), kw = (float)(c1 - c0);
+        const float nump = num / kh / kw, denp = den / kh / kw;
+        const float z = denp > 0.5f ? nump / fmax_(denp, 1e-6f) : 0.0f;
+        const float y = log_f32(fmax_(ld, 1e-3f)) - log_f32(fmax_(z, 1e-3f));
+        const bool m = cfd >= 2.0f && ld > 0.0f && z > 0.0f;
+        y_out[base + n] = y;
+        m_out[base + n] = m ? 1 : 0;
+        if (m) {
+            float a[kGaugeMaxK];
+            gauge_basis(linspace_at(ow, w), linspace_at(oh, h), a);
+            gauge_add<K>(a, y, 1.0f, G);
+        }
+    }
+    gauge_publish<K>(G, partials + ((int64_t)b * nblk + blockIdx.x) * kGaugeVals);
+}
+
+template <int K>
+__global__ __launch_bounds__(kGaugeBlk) void gauge_resid_k(int it, const float* __restrict__ y_all,
+                                                           const uint8_t* __restrict__ m_all, int h, int w, int nblk,
+                                                           const double* __restrict__ partials,
+                                                           GaugeState* __restrict__ st, uint32_t* __restrict__ r_all,
+                                                           uint32_t* __restrict__ hist) {
+    __shared__ uint32_t s_h[kGaugeBins];
+    __shared__ uint32_t s_below;
+    const int b = blockIdx.y, tid = threadIdx.x;
+    float c[kGaugeMaxK];
+    int count;
+    bool ok = gauge_solve<K>(partials + (int64_t)b * nblk * kGaugeVals, nblk, c, count);
+    if (it > 0) ok = ok && st[b].valid[(it - 1) & 1] != 0;
+    if (blockIdx.x == 0 && tid == 0) {
+        st[b].valid[it & 1] = ok ? 1 : 0;
+        st[b].rank = ok ? (uint32_t)((count - 1) / 2) : 0u;  // torch.median: the lower middle element
+        st[b].listed = 0u;
+    }
+    if (!ok) return;
+    for (int i = tid; i < kGaugeBins; i += kGaugeBlk) s_h[i] = 0u;
+    if (tid == 0) s_below = 0u;
+    __syncthreads();
     const int64_t N = (int64_t)h * w, base = (int64_t)b * N;
     int64_t n0, n1;
     gauge_range(N, nblk, blockIdx.x, n0, n1);
-    double G[NG + K + 1];
-#pragma unroll
-    for (int k = 0; k < NG + K + 1; ++k) G[k] = 0.0;
+    uint32_t below = 0u;
     for (int64_t n = n0 + tid; n < n1; n += kGaugeBlk) {
         if (!m_all[base + n]) continue;
         float a[kGaugeMaxK];
         const int iy = (int)(n / w), ix = (int)(n - (int64_t)iy * w);
         gauge_basis(linspace_at(ix, w), linspace_at(iy, h), a);
-        const float wn = first ? 1.0f : w_all[base + n];
-        float wa[K];
+        float p = 0.0f;
 #pragma unroll
-        for (int k = 0; k < K; ++k) wa[k] = a[k] * wn;
-        const float wy = y_all[base + n] * wn;
-        int e = 0;
-#pragma unroll
-        for (int i = 0; i < K; ++i)
-#pragma unroll
-            for (int j = i; j < K; ++j) G[e++] += (double)wa[i] * (double)wa[j];
-#pragma unroll
-        for (int i = 0; i < K; ++i) G[NG + i] += (double)wa[i] * (double)wy;
-        G[NG + K] += 1.0;
+        for (int k = 0; k < K; ++k) p = p + a[k] * c[k];
+        const uint32_t v = __float_as_uint(fabsf(y_all[base + n] - p));
+        r_all[base + n] = v;
+        const uint32_t d = v - kGaugeLow;
+        if (v < kGaugeLow)
+            ++below;
+        else if (d < ((uint32_t)kGaugeBins << kGaugeShift))
+            atomicAdd(&s_h[d >> kGaugeShift], 1u);
     }
-    const int wv = tid >> 6, lane = tid & 63;
-#pragma unroll
-    for (int k = 0; k < NG + K + 1; ++k) {
-        double v = G[k];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0) s_red[wv][k] = v;
-    }
+    below = wave_incl_scan_u32(below);
+    if ((tid & 63) == 63 && below) atomicAdd(&s_below, below);
     __syncthreads();
-    if (tid < NG + K + 1) {
-        double v = 0.0;
-        for (int q = 0; q < kGaugeBlk / 64; ++q) v += s_red[q][tid];
-        partials[((int64_t)b * nblk + blockIdx.x) * kGaugeVals + tid] = v;
-    }
+    uint32_t* hg = hist + (int64_t)b * kGaugeHist;
+    uint32_t v[kGaugeBins / kGaugeBlk];
+#pragma unroll
+    for (int k = 0; k < kGaugeBins / kGaugeBlk; ++k) v[k] = s_h[k * kGaugeBlk + tid];
+#pragma unroll
+    for (int k = 0; k < kGaugeBins / kGaugeBlk; ++k)
+        if (v[k]) atomicAdd(&hg[k * kGaugeBlk + tid], v[k]);
+    if (tid == 0 && s_below) atomicAdd(&hg[kGaugeBins], s_below);
 }
 
-// One wave per frame: the fixed-order reduction of the block partials, the count test, the solve (lane 0), and
-// the set-up of the median search; it also clears the frame's histogram for the first pass.
-template <int K>
-__global__ __launch_bounds__(64) void gauge_solve_k(const double* __restrict__ partials, int nblk, int first,
-                                                    GaugeState* __restrict__ st, float* __restrict__ coef,
-                                                    uint32_t* __restrict__ hist) {
-    constexpr int NG = K * (K + 1) / 2;
-    __shared__ double s_v[kGaugeVals];
-    const int b = blockIdx.x, lane = threadIdx.x;
-    for (int i = lane; i < kGaugeBins; i += 64) hist[(int64_t)b * kGaugeBins + i] = 0u;
-    if (!first && !st[b].valid) return;
-    if (lane < NG + K + 1) {
-        double v = 0.0;
-        for (int q = 0; q < nblk; ++q) v += partials[((int64_t)b * nblk + q) * kGaugeVals + lane];
-        s_v[lane] = v;
-    }
-    __syncthreads();
-    if (lane != 0) return;
-    const int count = (int)s_v[NG + K];
-    bool okk = count >= kGaugeMinPoints;  // v3.py:174-175: the frame keeps the correction 1
-    double A[K][K + 1];
-    {
-        int e = 0;
-        for (int i = 0; i < K; ++i) {
-            for (int j = i; j < K; ++j) {
-                A[i][j] = A[j][i] = s_v[e];
-                ++e;
-            }
-            A[i][K] = s_v[NG + i];
-        }
-    }
-    // Gaussian elimination with partial pivoting on [G | g]
-    for (int c = 0; c < K && okk; ++c) {
-        int p = c;
-        for (int r = c + 1; r < K; ++r)
-            if (fabs(A[r][c]) > fabs(A[p][c])) p = r;
-        if (!(fabs(A[p][c]) > 0.0)) {
-            okk = false;
-            break;
-        }
-        if (p != c)
-            for (int k = 0; k <= K; ++k) {
-                const double t = A[c][k];
-                A[c][k] = A[p][k];
-                A[p][k] = t;
-            }
-        for (int r = c + 1; r < K; ++r) {
-            const double f = A[r][c] / A[c][c];
-            for (int k = c; k <= K; ++k) A[r][k] -= f * A[c][k];
-        }
-    }
-    double x[K];
-    for (int c = K - 1; c >= 0 && okk; --c) {
-        double s = A[c][K];
-        for (int k = c + 1; k < K; ++k) s -= A[c][k] * x[k];
-        x[c] = s / A[c][c];
-    }
-    float cf[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int k = 0; k < K && okk; ++k) {
-        cf[k] = (float)x[k];
-        okk = __builtin_isfinite(cf[k]);
-    }
-    cf[7] = okk ? 1.0f : 0.0f;
-    for (int k = 0; k < 8; ++k) coef[b * 8 + k] = okk || k == 7 ? cf[k] : 0.0f;
-    GaugeState g;
-    g.prefix = 0u;
-    g.rank = okk ? (uint32_t)((count - 1) / 2) : 0u;  // torch.median: the lower middle element
-    g.count = count;
-    g.valid = okk ? 1 : 0;
-    st[b] = g;
-}
-
-// Radix pass `pass` (bits 31..21, 20..10, 9..0) of the median of |y - A c| over the confident pixels; pass 0 also
-// computes and keeps the residual bits (fp32, terms in basis order).
-template <int K>
-__global__ __launch_bounds__(kGaugeBlk) void gauge_hist_k(int pass, const float* __restrict__ y_all,
-                                                          const uint8_t* __restrict__ m_all, int h, int w,
-                                                          const float* __restrict__ coef,
-                                                          const GaugeState* __restrict__ st, int nblk,
-                                                          uint32_t* __restrict__ r_all, uint32_t* __restrict__ hist) {
-    __shared__ uint32_t s_h[kGaugeBins];
-    const int b = blockIdx.y, tid = threadIdx.x;
-    if (!st[b].valid) return;
-    for (int i = tid; i < kGaugeBins; i += kGaugeBlk) s_h[i] = 0u;
-    __syncthreads();
-    const int64_t N = (int64_t)h * w, base = (int64_t)b * N;
-    int64_t n0, n1;
-    gauge_range(N, nblk, blockIdx.x, n0, n1);
-    const int sh = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
-    const uint32_t bmask = pass == 2 ? 0x3ffu : 0x7ffu;
-    const uint32_t hmask = pass == 0 ? 0u : (pass == 1 ? 0xffe00000u : 0xfffffc00u);
-    const uint32_t prefix = st[b].prefix;
-    float c[kGaugeMaxK];
-#pragma unroll
-    for (int k = 0; k < kGaugeMaxK; ++k) c[k] = k < K ? coef[b * 8 + k] : 0.0f;
-    for (int64_t n = n0 + tid; n < n1; n += kGaugeBlk) {
-        if (!m_all[base + n]) continue;
-        uint32_t v;
-        if (pass == 0) {
-            float a[kGaugeMaxK];
-            const int iy = (int)(n / w), ix = (int)(n - (int64_t)iy * w);
-            gauge_basis(linspace_at(ix, w), linspace_at(iy, h), a);
-            float p = 0.0f;
-#pragma unroll
-            for (int k = 0; k < K; ++k) p = p + a[k] * c[k];
-            v = __float_as_uint(fabsf(y_all[base + n] - p));
-            r_all[base + n] = v;
-        } else {
-            v = r_all[base + n];
-        }
-        if ((v & hmask) == prefix) atomicAdd(&s_h[(v >> sh) & bmask], 1u);
-    }
-    __syncthreads();
-    uint32_t* hg = hist + (int64_t)b * kGaugeBins;
-    for (int i = tid; i < kGaugeBins; i += kGaugeBlk)
-        if (s_h[i]) atomicAdd(&hg[i], s_h[i]);
-}
-
-// One block per frame: the bucket of the pass that holds the rank; clears the histogram for the next pass.
-__global__ __launch_bounds__(kGaugeBlk) void gauge_select_k(int pass, GaugeState* __restrict__ st,
-                                                            uint32_t* __restrict__ hist) {
-    __shared__ uint32_t s_h[kGaugeBins];
-    __shared__ uint32_t s_part[kGaugeBlk];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    uint32_t* hg = hist + (int64_t)b * kGaugeBins;
-    const bool valid = st[b].valid != 0;
-    constexpr int PER = kGaugeBins / kGaugeBlk;  // 8 bins per thread
+// The bin of 2048 holding the rank-th (0-based) of the counted elements, in every thread of the block: its index and the
+// count before it; -1 when the rank lies at or past their total. `v`: the thread's 8 consecutive bins.
+__device__ inline int gauge_find(const uint32_t (&v)[kGaugeBins / kGaugeBlk], uint32_t rank, uint32_t& before) {
+    constexpr int PER = kGaugeBins / kGaugeBlk;
+    __shared__ uint32_t s_w[kGaugeBlk / 64];
+    __shared__ int s_bin;
+    __shared__ uint32_t s_before;
+    const int tid = threadIdx.x;
     uint32_t sum = 0u;
-    for (int k = 0; k < PER; ++k) {
-        const uint32_t v = valid ? hg[tid * PER + k] : 0u;
-        s_h[tid * PER + k] = v;
-        sum += v;
-    }
-    s_part[tid] = sum;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) sum += v[k];
+    const uint32_t inc = wave_incl_scan_u32(sum);
+    if ((tid & 63) == 63) s_w[tid >> 6] = inc;
+    if (tid == 0) s_bin = -1;
     __syncthreads();
-    for (int i = tid; i < kGaugeBins; i += kGaugeBlk) hg[i] = 0u;
-    if (!valid || tid != 0) return;
-    const int sh = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
-    const int nb = pass == 2 ? 1024 : 2048;
-    uint32_t k = st[b].rank, cum = 0u;
-    int t = 0;
-    while (t < kGaugeBlk - 1 && cum + s_part[t] <= k) cum += s_part[t++];
-    int bkt = t * PER;
-    for (; bkt < nb - 1; ++bkt) {
-        if (cum + s_h[bkt] > k) break;
-        cum += s_h[bkt];
+    uint32_t cum = inc - sum;
+    for (int q = 0; q < (tid >> 6); ++q) cum += s_w[q];
+    if (cum <= rank && rank < cum + sum) {
+        int at = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const bool past = at == k && cum + v[k] <= rank;
+            cum += past ? v[k] : 0u;
+            at += past ? 1 : 0;
+        }
+        s_bin = tid * PER + at;
+        s_before = cum;
     }
-    st[b].prefix |= (uint32_t)bkt << sh;
-    st[b].rank = k - cum;
+    __syncthreads();
+    before = s_before;
+    const int bin = s_bin;
+    __syncthreads();
+    return bin;
 }
 
-__global__ __launch_bounds__(kGaugeBlk) void gauge_weights_k(const uint8_t* __restrict__ m_all, int h, int w,
-                                                             const GaugeState* __restrict__ st, int nblk,
-                                                             const uint32_t* __restrict__ r_all,
-                                                             float* __restrict__ w_all) {
-    const int b = blockIdx.y, tid = threadIdx.x;
-    if (!st[b].valid) return;
-    const int64_t N = (int64_t)h * w, base = (int64_t)b * N;
+__global__ __launch_bounds__(kGaugeBlk) void gauge_pick_k(int it, const uint8_t* __restrict__ m_all, int64_t N, int nblk,
+                                                          GaugeState* __restrict__ st,
+                                                          const uint32_t* __restrict__ r_all,
+                                                          const uint32_t* __restrict__ hist,
+                                                          uint32_t* __restrict__ list) {
+    constexpr int PER = kGaugeBins / kGaugeBlk;
+    const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    if (!st[b].valid[it & 1]) return;
+    const uint32_t* hg = hist + (int64_t)b * kGaugeHist;
+    const uint32_t below = hg[kGaugeBins], rank = st[b].rank;
+    uint32_t v[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) v[k] = hg[tid * PER + k];
+    uint32_t before = 0u, lo = 0u, hi = kGaugeLow - 1u, lrank = rank;
+    if (rank >= below) {
+        const int bin = gauge_find(v, rank - below, before);
+        if (bin >= 0) {
+            lo = kGaugeLow + ((uint32_t)bin << kGaugeShift);
+            hi = lo + ((1u << kGaugeShift) - 1u);
+            lrank = rank - below - before;
+        } else {  // above the bins: their total lies before it
+            uint32_t sum = 0u;
+            for (int k = 0; k < kGaugeBins; ++k) sum += hg[k];
+            lo = kGaugeLow + ((uint32_t)kGaugeBins << kGaugeShift);
+            hi = 0x7fffffffu;
+            lrank = rank - below - sum;
+        }
+    }
+    if (blockIdx.x == 0 && tid == 0) {
+        st[b].key_lo = lo;
+        st[b].key_hi = hi;
+        st[b].list_rank = lrank;
+    }
+    const int64_t base = (int64_t)b * N;
     int64_t n0, n1;
     gauge_range(N, nblk, blockIdx.x, n0, n1);
-    const float med = __uint_as_float(st[b].prefix);
-    const float sc = 1.4826f * med + 1e-4f;
-    for (int64_t n = n0 + tid; n < n1; n += kGaugeBlk) {
-        if (!m_all[base + n]) continue;
-        w_all[base + n] = fmin_((2.0f * sc) / fmax_(__uint_as_float(r_all[base + n]), 1e-6f), 1.0f);
+    for (int64_t n = n0; n < n1; n += kGaugeBlk) {  // whole waves: the listed of a wave take one atomic
+        const bool in = n + tid < n1 && m_all[base + n + tid] != 0;
+        const uint32_t key = in ? r_all[base + n + tid] : 0xffffffffu;
+        const bool hit = key >= lo && key <= hi;
+        const uint64_t mask = __ballot(hit);
+        if (mask == 0) continue;
+        uint32_t at = 0u;
+        if (lane == 0) at = atomicAdd(&st[b].listed, (uint32_t)__popcll(mask));
+        at = (uint32_t)__builtin_amdgcn_readlane((int)at, 0);
+        if (hit)
+            list[base + at + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = key;
     }
 }
 
 template <int K>
-__global__ __launch_bounds__(256) void gauge_apply_k(const float* __restrict__ coef, int H, int W, int64_t n_out,
-                                                     float* __restrict__ out) {
-    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (q >= n_out) return;
-    const int64_t plane = (int64_t)H * W;
-    const int64_t b = q / plane;
-    const int rem = (int)(q - b * plane);
-    const int i = rem / W, j = rem - i * W;
-    const float* c = coef + b * 8;
-    if (c[7] == 0.0f) {
-        out[q] = 1.0f;
-        return;
-    }
-    float a[kGaugeMaxK];
-    gauge_basis(linspace_at(j, W), linspace_at(i, H), a);
-    float p = 0.0f;
+__global__ __launch_bounds__(kGaugeBlk) void gauge_sums_k(int it, const float* __restrict__ y_all,
+                                                          const uint8_t* __restrict__ m_all, int h, int w, int nblk,
+                                                          const GaugeState* __restrict__ st,
+                                                          const uint32_t* __restrict__ r_all,
+                                                          const uint32_t* __restrict__ list,
+                                                          uint32_t* __restrict__ hist,
+                                                          double* __restrict__ partials) {
+    constexpr int PER = kGaugeBins / kGaugeBlk;
+    __shared__ uint32_t s_h[kGaugeBins];
+    __shared__ alignas(16) uint32_t s_keys[kGaugeList];
+    __shared__ uint32_t s_med;
+    const int b = blockIdx.y, tid = threadIdx.x;
+    if (!st[b].valid[it & 1]) return;
+    for (int i = blockIdx.x * kGaugeBlk + tid; i < kGaugeHist; i += nblk * kGaugeBlk) hist[(int64_t)b * kGaugeHist + i] = 0u;
+    const int64_t N = (int64_t)h * w, base = (int64_t)b * N;
+    // ---- the median among the listed keys (their order in the list varies; the median does not)
+    const uint32_t L = st[b].listed, lo = st[b].key_lo;
+    uint32_t rank = st[b].list_rank;
+    const bool held = L <= (uint32_t)kGaugeList;
+    if (held)
+        for (uint32_t i = tid; i < L; i += kGaugeBlk) s_keys[i] = list[base + i];
+    uint32_t med = lo;
+    if (L <= (uint32_t)kGaugeBlk) {  // each thread ranks one key against all
+        if (tid == 0) s_med = lo;
+        const uint32_t L4 = (L + 3u) & ~3u;
+        if ((uint32_t)tid >= L && (uint32_t)tid < L4) s_keys[tid] = 0xffffffffu;
+        __syncthreads();
+        const uint32_t key = (uint32_t)tid < L ? s_keys[tid] : 0xffffffffu;
+        uint32_t less = 0u, eq = 0u;
+#pragma unroll 4
+        for (uint32_t i = 0; i < L4; i += 4) {
+            const uint4 q = *(const uint4*)&s_keys[i];
+            less += (q.x < key ? 1u : 0u) + (q.y < key ? 1u : 0u) + (q.z < key ? 1u : 0u) + (q.w < key ? 1u : 0u);
+            eq += (q.x == key ? 1u : 0u) + (q.y == key ? 1u : 0u) + (q.z == key ? 1u : 0u) + (q.w == key ? 1u : 0u);
+        }
+        if ((uint32_t)tid < L && less <= rank && rank < less + eq) s_med = key;  // equal keys write equal values
+        __syncthreads();
+        med = s_med;
+    } else {  // radix select over key - lo, 11 bits a pass
+        const uint32_t range = st[b].key_hi - lo;
+        uint32_t prefix = 0u, pmask = 0u;
+        for (int top = 32 - __builtin_clz(range); top > 0;) {
+            const int width = top < 11 ? top : 11, sh = top - width;
+            const uint32_t dmask = (1u << width) - 1u;
+            __syncthreads();
+            for (int i = tid; i < kGaugeBins; i += kGaugeBlk) s_h[i] = 0u;
+            __syncthreads();
+            for (uint32_t i = tid; i < L; i += kGaugeBlk) {
+                const uint32_t k = (held ? s_keys[i] : list[base + i]) - lo;
+                if ((k & pmask) == prefix) atomicAdd(&s_h[(k >> sh) & dmask], 1u);
+            }
+            __syncthreads();
+            uint32_t v[PER], before;
 #pragma unroll
-    for (int k = 0; k < K; ++k) p = p + a[k] * c[k];
-    out[q] = exp_f32(p);
+            for (int k = 0; k < PER; ++k) v[k] = s_h[tid * PER + k];
+            const int bin = gauge_find(v, rank, before);
+            prefix |= (uint32_t)bin << sh;
+            pmask |= dmask << sh;
+            rank -= before;
+            top = sh;
+        }
+        med = lo + prefix;
+    }
+    const float sc = 1.4826f * __uint_as_float(med) + 1e-4f;
+    int64_t n0, n1;
+    gauge_range(N, nblk, blockIdx.x, n0, n1);
+    double G[K * (K + 1) / 2 + K + 1] = {};
+    for (int64_t n = n0 + tid; n < n1; n += kGaugeBlk) {
+        if (!m_all[base + n]) continue;
+        float a[kGaugeMaxK];
+        const int iy = (int)(n / w), ix = (int)(n - (int64_t)iy * w);
+        gauge_basis(linspace_at(ix, w), linspace_at(iy, h), a);
+        const float wn = fmin_((2.0f * sc) / fmax_(__uint_as_float(r_all[base + n]), 1e-6f), 1.0f);
+        gauge_add<K>(a, y_all[base + n], wn, G);
+    }
+    gauge_publish<K>(G, partials + ((int64_t)b * nblk + blockIdx.x) * kGaugeVals);
+}
+
+// Solves the last round's system (each block) and applies it: grid.x blocks walk a frame's pixels.
+template <int K>
+__global__ __launch_bounds__(kGaugeBlk) void gauge_apply_k(int it, const double* __restrict__ partials, int nblk,
+                                                           const GaugeState* __restrict__ st, int H, int W,
+                                                           float* __restrict__ coef, float* __restrict__ out) {
+    const int b = blockIdx.y, tid = threadIdx.x;
+    float c[kGaugeMaxK];
+    int count;
+    bool ok = gauge_solve<K>(partials + (int64_t)b * nblk * kGaugeVals, nblk, c, count);
+    if (it > 0) ok = ok && st[b].valid[(it - 1) & 1] != 0;
+    if (blockIdx.x == 0 && tid < 8) coef[b * 8 + tid] = 0.0f;
+    if (blockIdx.x == 0 && tid == 0 && ok) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) coef[b * 8 + k] = c[k];
+        coef[b * 8 + 7] = 1.0f;
+    }
+    const uint32_t plane = (uint32_t)(H * W);  // below 2^31
+    float* const ob = out + (int64_t)b * plane;
+    for (uint32_t q = blockIdx.x * kGaugeBlk + tid; q < plane; q += gridDim.x * kGaugeBlk) {
+        const int i = (int)(q / (uint32_t)W), j = (int)(q - (uint32_t)i * (uint32_t)W);
+        float a[kGaugeMaxK];
+        gauge_basis(linspace_at(j, W), linspace_at(i, H), a);
+        float p = 0.0f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) p = p + a[k] * c[k];
+        ob[q] = ok ? exp_f32(p) : 1.0f;
+    }
 }
 
 }  // namespace pmg
 
 using namespace pmg;
 
+// Blocks per frame: two pixels a thread up to 256 blocks (every block of the next kernel reads all their partials).
 static int gauge_blocks(int64_t N) {
-    const int64_t nb = (N + 1023) / 1024;
+    const int64_t nb = (N + 2 * kGaugeBlk - 1) / (2 * kGaugeBlk);
     return (int)(nb < 1 ? 1 : (nb > kGaugeMaxBlocks ? kGaugeMaxBlocks : nb));
 }
 
 template <int K>
-static int gauge_rounds(const float* y, const uint8_t* m, int B, int h, int w, int iters, float* wt, uint32_t* rb,
-                        double* partials, uint32_t* hist, GaugeState* st, float* coef, hipStream_t s) {
+static int gauge_run(const float* depth, const float* lidar, const float* conf, int B, int H, int W, int h, int w,
+                     int iters, float* y, uint8_t* m, uint32_t* rb, uint32_t* list, double* partials, uint32_t* hist,
+                     GaugeState* st, float* coef, float* corr, hipStream_t s) {
     const int nblk = gauge_blocks((int64_t)h * w);
-    const dim3 grid((unsigned)nblk, (unsigned)B);
-    for (int it = 0; it < iters; ++it) {
-        const int first = it == 0;
-        hipLaunchKernelGGL(gauge_sums_k<K>, grid, dim3(kGaugeBlk), 0, s, y, m, wt, h, w, first, st, nblk, partials);
+    const dim3 grid((unsigned)nblk, (unsigned)B), blk(kGaugeBlk);
+    hipLaunchKernelGGL(gauge_inputs_k<K>, grid, blk, 0, s, depth, lidar, conf, H, W, h, w, nblk, y, m, hist, partials);
+    if (int e = check_launch("gauge_inputs_k")) return e;
+    for (int it = 0; it + 1 < iters; ++it) {  // (the last round's weights are never used)
+        hipLaunchKernelGGL(gauge_resid_k<K>, grid, blk, 0, s, it, y, m, h, w, nblk, partials, st, rb, hist);
+        if (int e = check_launch("gauge_resid_k")) return e;
+        hipLaunchKernelGGL(gauge_pick_k, grid, blk, 0, s, it, m, (int64_t)h * w, nblk, st, rb, hist, list);
+        if (int e = check_launch("gauge_pick_k")) return e;
+        hipLaunchKernelGGL(gauge_sums_k<K>, grid, blk, 0, s, it, y, m, h, w, nblk, st, rb, list, hist, partials);
         if (int e = check_launch("gauge_sums_k")) return e;
-        hipLaunchKernelGGL(gauge_solve_k<K>, dim3(B), dim3(64), 0, s, partials, nblk, first, st, coef, hist);
-        if (int e = check_launch("gauge_solve_k")) return e;
-        if (it + 1 == iters) break;  // the last weights are never used
-        for (int pass = 0; pass < 3; ++pass) {
-            hipLaunchKernelGGL(gauge_hist_k<K>, grid, dim3(kGaugeBlk), 0, s, pass, y, m, h, w, coef, st, nblk, rb,
-                               hist);
-            if (int e = check_launch("gauge_hist_k")) return e;
-            hipLaunchKernelGGL(gauge_select_k, dim3(B), dim3(kGaugeBlk), 0, s, pass, st, hist);
-            if (int e = check_launch("gauge_select_k")) return e;
-        }
-        hipLaunchKernelGGL(gauge_weights_k, grid, dim3(kGaugeBlk), 0, s, m, h, w, st, nblk, rb, wt);
-        if (int e = check_launch("gauge_weights_k")) return e;
     }
-    return PMG_OK;
+    // every block repeats the solve (2 us), so a frame gets at most 512 blocks, two per CU
+    const int64_t na = ((int64_t)H * W + kGaugeBlk - 1) / kGaugeBlk;
+    hipLaunchKernelGGL(gauge_apply_k<K>, dim3((unsigned)(na < 512 ? na : 512), (unsigned)B), blk, 0, s, iters - 1,
+                       partials, nblk, st, H, W, coef, corr);
+    return check_launch("gauge_apply_k");
 }
 
 extern "C" {
@@ -377,7 +520,7 @@ size_t pmg_gauge_poly_workspace_bytes(int B, int h, int w) {
     const size_t n = (size_t)B * h * w;
     const int nblk = gauge_blocks((int64_t)h * w);
     return align256(n * 4) + align256(n) + align256(n * 4) + align256(n * 4) +
-           align256((size_t)B * nblk * kGaugeVals * sizeof(double)) + align256((size_t)B * kGaugeBins * 4) +
+           align256((size_t)B * nblk * kGaugeVals * sizeof(double)) + align256((size_t)B * kGaugeHist * 4) +
            align256((size_t)B * sizeof(GaugeState));
 }
 
@@ -391,35 +534,26 @@ int pmg_gauge_poly(const float* depth, int B, int H, int W, const float* lidar, 
     PMG_REQUIRE(iters >= 1 && iters <= 64, "iters must be in [1, 64]");
     PMG_REQUIRE(workspace && workspace_bytes >= pmg_gauge_poly_workspace_bytes(B, h, w), "workspace too small");
     hipStream_t s = (hipStream_t)stream;
-    const int64_t n_lr = (int64_t)B * h * w, n_out = (int64_t)B * H * W;
+    const int64_t n_lr = (int64_t)B * h * w;
     const int nblk = gauge_blocks((int64_t)h * w);
     uint8_t* p = (uint8_t*)workspace;
     float* y = (float*)p;
     p += align256((size_t)n_lr * 4);
     uint8_t* m = p;
     p += align256((size_t)n_lr);
-    float* wt = (float*)p;
+    uint32_t* list = (uint32_t*)p;
     p += align256((size_t)n_lr * 4);
     uint32_t* rb = (uint32_t*)p;
     p += align256((size_t)n_lr * 4);
     double* partials = (double*)p;
     p += align256((size_t)B * nblk * kGaugeVals * sizeof(double));
     uint32_t* hist = (uint32_t*)p;
-    p += align256((size_t)B * kGaugeBins * 4);
+    p += align256((size_t)B * kGaugeHist * 4);
     GaugeState* st = (GaugeState*)p;
-    hipLaunchKernelGGL(gauge_inputs_k, dim3((unsigned)((n_lr + 255) / 256)), dim3(256), 0, s, depth, lidar, conf, H, W,
-                       h, w, n_lr, y, m);
-    if (int e = check_launch("gauge_inputs_k")) return e;
-    if (degree >= 2) {
-        if (int e = gauge_rounds<6>(y, m, B, h, w, iters, wt, rb, partials, hist, st, coef, s)) return e;
-        hipLaunchKernelGGL(gauge_apply_k<6>, dim3((unsigned)((n_out + 255) / 256)), dim3(256), 0, s, coef, H, W, n_out,
-                           corr);
-    } else {
-        if (int e = gauge_rounds<3>(y, m, B, h, w, iters, wt, rb, partials, hist, st, coef, s)) return e;
-        hipLaunchKernelGGL(gauge_apply_k<3>, dim3((unsigned)((n_out + 255) / 256)), dim3(256), 0, s, coef, H, W, n_out,
-                           corr);
-    }
-    return check_launch("gauge_apply_k");
+    return degree >= 2 ? gauge_run<6>(depth, lidar, conf, B, H, W, h, w, iters, y, m, rb, list, partials, hist, st, coef,
+                                      corr, s)
+                       : gauge_run<3>(depth, lidar, conf, B, H, W, h, w, iters, y, m, rb, list, partials, hist, st, coef,
+                                      corr, s);
 }
 
 }  // extern "C"

@@ -114,3 +114,25 @@ def test_gauge_three_frames_degree3_odd_grid(gpu):
     lidar = np.concatenate([m[1] for m in maps])
     conf = np.concatenate([m[2] for m in maps])
     _check(depth, lidar, conf, degree=3)
+
+
+@pytest.mark.parametrize("case,hw", [("exact", (120, 160)), ("wide", (61, 83)), ("half_ties", (97, 131)), ("one_block", (16, 16)),
+                                     ("many", (300, 470))])
+def test_gauge_median_paths(gpu, case, hw):
+    """The median's ways: all residuals below the histogram's range and more of them than a block's list holds ("exact":
+    a constant gauge), above it ("wide": a log-gauge noise of about 1), most of one value ("half_ties"), a frame of one
+    block, and one of 256 blocks whose medians' bins hold several hundred."""
+    announce(f"gauge median paths: {case} {hw}")
+    h, w = hw
+    rng = np.random.default_rng(h)
+    lidar = rng.uniform(0.5, 5.0, (2, h, w)).astype(np.float32)
+    depth = lidar.copy()
+    if case == "exact":
+        lidar = lidar * np.float32(2.0)
+    elif case == "wide":
+        lidar = (lidar * np.exp(rng.normal(0, 1.0, lidar.shape))).astype(np.float32)
+    elif case == "half_ties":
+        lidar = np.where(rng.random(lidar.shape) < 0.4, lidar * np.float32(1.25), lidar).astype(np.float32)
+    else:
+        lidar = (lidar * np.exp(rng.normal(0, 0.02, lidar.shape))).astype(np.float32)
+    _check(depth, lidar, np.full((2, h, w), 2.0, np.float32))
