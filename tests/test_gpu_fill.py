@@ -49,6 +49,17 @@ def test_fill_random(gpu, h, w, hole):
     _check(d[None], c[None], gpu)
 
 
+@pytest.mark.parametrize("h,w,hole", [(63, 40, 0.99), (64, 513, 0.999), (129, 30, 0.995), (300, 511, 0.9995), (321, 1, 0.98)])
+def test_fill_holes_over_several_words(gpu, h, w, hole):
+    """Holes of more than 64 rows (a column's nearest row lies several words away, above or below), rows at the edges of the
+    64-row words, widths around the row kernel's block sizes."""
+    announce(f"nearest_fill {h}x{w} hole={hole}")
+    rng = np.random.default_rng(h * 1000 + w + 1)
+    d, c = _case(rng, h, w, hole)
+    d[h // 2, w // 2] = 1.5
+    _check(d[None], c[None], gpu)
+
+
 def test_fill_tie_lattices_and_batch(gpu):
     announce("nearest_fill lattices, batch of 5 incl. empty and full images")
     h, w = 61, 77
