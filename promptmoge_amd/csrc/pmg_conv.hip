@@ -311,6 +311,30 @@ __device__ inline void store_tile_codes(const ConvArgs& a, const v4i (&acc)[T][N
     }
 }
 
+// Epilogue of the float kernels: channels n .. n + 3 of one row (accumulators, their biases) at element o of the output.
+template <int EPI>
+__device__ inline void store_float4(const ConvArgs& a, int64_t o, const v4f& acc, const float* bias) {
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        y[i] = acc[i];
+        if constexpr (EPI != PMG_EPI_ACC) {
+            if (a.bias) y[i] = y[i] + bias[i];
+        }
+    }
+    if constexpr (EPI == PMG_EPI_SILU) {
+        float h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = silu_fast(y[i]);
+        store_half4(h, (_Float16*)a.out + o);
+    } else if constexpr (EPI == PMG_EPI_R) {
+        const v4f sk = *(const v4f*)(a.skip + o);
+        *(v4f*)((float*)a.out + o) = v4f{y[0] + sk[0], y[1] + sk[1], y[2] + sk[2], y[3] + sk[3]};
+    } else {
+        *(v4f*)((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
+    }
+}
+
 // Host-sized generic-map launches deal groups of kXcdGroup consecutive chunks round-robin over the 8 XCDs (block b
 // runs on XCD b % 8): neighbouring chunks (rows that share neighbours) stay on one XCD's L2, and the work evens out
 // where it varies along the row order (rows sorted by tap mask; measured at C = 128 on the 1M-voxel surface set:
@@ -606,26 +630,7 @@ __global__ __launch_bounds__(kG2Threads, 1) void spconv_g2_k(ConvArgs a) {
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
                     const int64_t o = (int64_t)m * Co + n0 + 16 * j + 4 * g;
-                    float y[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        y[i] = acc[t][j][i];
-                        if constexpr (EPI != PMG_EPI_ACC) {
-                            if (a.bias) y[i] = y[i] + s_k[1][16 * j + 4 * g + i];
-                        }
-                    }
-                    if constexpr (EPI == PMG_EPI_SILU) {
-                        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                        h4 hv;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) hv[i] = (_Float16)silu_fast(y[i]);
-                        *(h4*)((_Float16*)a.out + o) = hv;
-                    } else if constexpr (EPI == PMG_EPI_R) {
-                        const v4f sk = *(const v4f*)(a.skip + o);
-                        *(v4f*)((float*)a.out + o) = v4f{y[0] + sk[0], y[1] + sk[1], y[2] + sk[2], y[3] + sk[3]};
-                    } else {
-                        *(v4f*)((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
-                    }
+                    store_float4<EPI>(a, o, acc[t][j], s_k[1] + 16 * j + 4 * g);
                 }
             }
         } else if constexpr (EPI == PMG_EPI_Q || EPI == PMG_EPI_QLIN) {
@@ -670,37 +675,50 @@ __global__ __launch_bounds__(kG2Threads, 1) void spconv_g2_k(ConvArgs a) {
 // their MFMAs and the map indices two taps before that. NWV waves per block (NWV = 16: four per SIMD, fewer
 // registers each): each wave spends most of a tap waiting for its gathers, so more waves and deeper rings keep
 // more of them in flight.
-template <int C, int EPI, int T = kG2Tiles, int PF = 1, int RS = 2, int NWV = kG2Waves>
+//
+// With NB < C / 16 the block holds the weights of a slice of 16 NB output channels, one slice per blockIdx.y, and
+// every slice gathers the rows again: fp16 / bf16 C = 64 in two slices of 32, fp32 C = 64 in four of 16 (108 KB each,
+// as is the whole of fp32 C = 32). Measured against spconv_g2_k, which stages these widths' weights tap by tap between
+// barriers: see launch_g2rf.
+template <int C, int EPI, int T = kG2Tiles, int PF = 1, int RS = 2, int NWV = kG2Waves, typename E = int8_t,
+          int NB = C / 16>
 __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
-    constexpr int NB = C / 16, KS = C / 64;
+    // row bytes, 64-byte K chunks (a last chunk of fewer bytes: the lane groups past it load zeros on both sides)
+    constexpr int RB = C * (int)sizeof(E), KS = (RB + 63) / 64, TAIL = RB % 64;
+    constexpr int NS = 16 * NB;                           // output channels of the block
     constexpr int NF = NB * KS;
+    typedef typename Acc<E>::type acc_t;
     constexpr int CHUNK = NWV * T * 16;
     constexpr int NTH = 64 * NWV;
     constexpr int GD = RS - 1;                 // gather distance in taps
     constexpr int UNR = RS % 2 == 0 ? RS : 2 * RS;  // steps per loop trip: the X ring (RS) and the index pair (2)
-    static_assert(C == 64, "resident weights: C = 64");
+    static_assert(RB % 16 == 0 && 27 * NF <= 112 && C % NS == 0, "resident weights: 16-byte chunks, at most 112 KB");
     static_assert(RS >= 2 && RS <= 4, "ring slots");
     __shared__ __attribute__((aligned(16))) v4i s_w[27 * NF * 64];
-    __shared__ float s_k[2][C];
+    __shared__ float s_k[2][NS];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
     const int S = (int)a.M;                     // map row stride (the capacity)
     const int M = a.m_dev ? (int)*a.m_dev : S;  // rows
     const int64_t ntile = (M + 15) >> 4;
     typedef const __attribute__((address_space(3))) v4i lds_v4i;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, (int)(a.M * C), kBufWord3);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, (int)(a.M * RB), kBufWord3);
     const __amdgpu_buffer_rsrc_t nr =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.nmap_t, (short)0, (int)(a.M * 27 * 4), kBufWord3);
-    for (int e = tid; e < 2 * C; e += NTH) {
-        const int q = e / C, n = e - (e / C) * C;
+    const int Co = NS == C ? C : a.Co;
+    const int n0 = NS == C ? 0 : (int)blockIdx.y * NS;  // first output channel of the block
+    for (int e = tid; e < 2 * NS; e += NTH) {
+        const int q = e / NS, n = e - (e / NS) * NS;
         const float* src = q == 0 ? a.w_scale : a.bias;
-        s_k[q][n] = src ? src[n] : 0.0f;
+        s_k[q][n] = src ? src[n0 + n] : 0.0f;
     }
     for (int e = tid; e < 27 * NF * 64; e += NTH) {
         const int f = e >> 6, l = e & 63;
         const int v = f / NF, js = f - (f / NF) * NF;
         const int j = js / KS, s2 = js - (js / KS) * KS;
-        s_w[e] = *(const v4i*)((const uint8_t*)a.w + ((l & 15) * 27) * C + 16 * (l >> 4) + ((16 * j * 27) + v) * C + 64 * s2);
+        const bool in = TAIL == 0 || 64 * s2 + 16 * (l >> 4) < RB;
+        s_w[e] = in ? *(const v4i*)(a.w + ((int64_t)(n0 + 16 * j + (l & 15)) * 27 + v) * RB + 64 * s2 + 16 * (l >> 4))
+                    : v4i{0, 0, 0, 0};
     }
     __syncthreads();
 
@@ -730,11 +748,11 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
             for (int o = 1; o < T; o <<= 1) mk |= __shfl_xor(mk, o, 64);
             wmask = (uint32_t)__builtin_amdgcn_readfirstlane((int)mk);
         }
-        v4i acc[T][NB];
+        acc_t acc[T][NB];
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int j = 0; j < NB; ++j) acc[t][j] = v4i{0, 0, 0, 0};
+            for (int j = 0; j < NB; ++j) acc[t][j] = acc_t{0, 0, 0, 0};
         auto idx_load = [&](int v, int (&id)[T]) {
             const int vo = (v < 27 ? v : 27) * S * 4;
 #pragma unroll
@@ -743,9 +761,11 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
         auto gather = [&](const int (&id)[T], v4i (&xs)[T][KS]) {
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const int off = id[t] >= 0 ? id[t] * C + 16 * g : (int)0x80000000;
+                const int off = id[t] >= 0 ? id[t] * RB + 16 * g : (int)0x80000000;
+                const int offt = TAIL == 0 || 16 * g < TAIL ? off : (int)0x80000000;  // of the last chunk
 #pragma unroll
-                for (int s2 = 0; s2 < KS; ++s2) xs[t][s2] = __builtin_amdgcn_raw_buffer_load_b128(xr, off, 64 * s2, 0);
+                for (int s2 = 0; s2 < KS; ++s2)
+                    xs[t][s2] = __builtin_amdgcn_raw_buffer_load_b128(xr, s2 == KS - 1 ? offt : off, 64 * s2, 0);
             }
         };
         auto mma_tap = [&](int v, const v4i (&xs)[T][KS]) {
@@ -764,7 +784,7 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int t = 0; t < T; ++t)
-                    acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur, xs[t][s2], acc[t][j], 0, 0, 0);
+                    mma(acc[t][j], cur, xs[t][s2], E{});
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -817,8 +837,8 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
                 tap(std::integral_constant<int, 5>{});
             }
         }
-        if constexpr (EPI == PMG_EPI_Q || EPI == PMG_EPI_QLIN) {
-            store_tile_codes<EPI, T, NB>(a, acc, s_k[0], s_k[1], orow, pos0, M, C, 0, g);
+        if constexpr (sizeof(E) == 1 && (EPI == PMG_EPI_Q || EPI == PMG_EPI_QLIN)) {
+            store_tile_codes<EPI, T, NB>(a, acc, s_k[0], s_k[1], orow, pos0, M, Co, n0, g);
             continue;
         }
 #pragma unroll
@@ -827,8 +847,10 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
             const int m = orow[t];
 #pragma unroll
             for (int j = 0; j < NB; ++j) {
-                const int64_t o = (int64_t)m * C + 16 * j + 4 * g;
-                if constexpr (EPI == PMG_EPI_ACC) {
+                const int64_t o = (int64_t)m * Co + n0 + 16 * j + 4 * g;
+                if constexpr (sizeof(E) != 1) {
+                    store_float4<EPI>(a, o, acc[t][j], s_k[1] + 16 * j + 4 * g);
+                } else if constexpr (EPI == PMG_EPI_ACC) {
                     *(v4i*)((int32_t*)a.out + o) = acc[t][j];
                 } else {
                     float y[4];
@@ -902,9 +924,8 @@ static int launch_g2(const ConvArgs& a, int epilogue, hipStream_t s) {
     }
 }
 
-// fp16 / bf16 / fp32 features, Ci = Co = C with rows of 64 - 1024 bytes: the weight-staged kernel on K chunks of 32
-// halves (v_mfma_f32_16x16x32_f16 / _bf16) or 16 floats (four v_mfma_f32_16x16x4f32), fp32 accumulators. Rows of
-// 256 bytes hold 16 tiles of accumulators per wave at T = 4, so they run T = 2; rows of 512 and 1024 bytes (fp16
+// fp16 / bf16 features, Ci = Co = C with rows of 128 - 1024 bytes: the weight-staged kernel on K chunks of 32 halves
+// (v_mfma_f32_16x16x32_f16 / _bf16), fp32 accumulators. Rows of 256 bytes hold 16 tiles of accumulators per wave at T = 4, so they run T = 2; rows of 512 and 1024 bytes (fp16
 // C = 256, 512) split the output channels into slices of 64 (blockIdx.y: a tap's weights fit the LDS buffers) and
 // run T = 2 and 1 (the gathered rows of the two ring slots fill the registers).
 template <typename E, int C>
@@ -932,13 +953,84 @@ static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
     return check_launch("spconv_g2_k");
 }
 
-// Whether the fp staged kernel takes this convolution: Ci = Co >= 32 with rows of 64 - 256 bytes (fp16 / bf16 32,
-// 64, 128; fp32 32, 64), or fp16 / bf16 rows of 512 or 1024 bytes (C = 256, 512: slices of 64 output channels),
-// 32-bit buffer offsets and aligned vectors.
+// Float features on resident weights (spconv_g2r_k): the slice of output channels whose 27 taps fit the LDS (108 KB at
+// most) -- all of C for 64-byte rows and fp32 C = 32, 32 channels for 16-bit C = 64, 16 for fp32 C = 64 and 16-bit
+// C = 128. Gathers three taps ahead (one tap ahead at T = 4: 58 us for T = 2's 40 at 77k rows, fp16 C = 64).
+constexpr int resident_nb(int C, int elt) {
+    const int ks = (C * elt + 63) / 64;
+    int nb = C / 16;
+    while (27 * nb * ks > 112 || C / 16 % nb != 0) --nb;
+    return nb;
+}
+template <typename E, int C, int T>
+static int launch_g2rf(const ConvArgs& a, int epilogue, hipStream_t s) {
+    static int cus = -1;
+    if (cus < 0) cus = num_cus();
+    constexpr int NB = resident_nb(C, (int)sizeof(E));
+    constexpr int CHUNK = kG2Waves * T * 16;
+    // one block per CU (its weights fill the LDS), the slices' blocks side by side, whole XCD rounds
+    int per = cus / (C / (16 * NB));
+    if (per >= 8) per -= per % 8;
+    const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
+    const dim3 grid((unsigned)(nchunk < per ? nchunk : per), (unsigned)(C / (16 * NB))), blk(kG2Threads);
+    switch (epilogue) {
+        case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_ACC, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a); break;
+        case PMG_EPI_BIAS: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_BIAS, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a); break;
+        case PMG_EPI_R:
+            if constexpr (sizeof(E) == 2) {
+                hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_R, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a);
+                break;
+            }
+            [[fallthrough]];
+        case PMG_EPI_SILU:
+            if constexpr (std::is_same<E, _Float16>::value) {
+                hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_SILU, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a);
+                break;
+            }
+            [[fallthrough]];
+        default: return fail(PMG_E_INVALID, "spconv: epilogue not available for this precision");
+    }
+    return check_launch("spconv_g2r_k");
+}
+
+// Ci = Co = C float features (g2f_fits): resident weights or staged ones, by the number of rows (a device-sized launch:
+// the rows its level is expected to hold). Measured on surface sets, one map, us, resident against staged:
+//   rows                2k         10k        30k        77k        184k       400k       1M
+//   16-bit C = 32     13 / 16    12 / 29    13 / 30    17 / 32    25 / 33    49 / 62    118 / 154
+//   16-bit C = 64     13 / 35    14 / 69    20 / 69    41 / 71    80 / 74   156 / 140   378 / 311
+//   16-bit C = 128    17 / 56    39 / 57    93 / 110  213 / 116   ..
+//   16-bit C = 48     11 / 20    11 / 21    21 / 26    40 / 54    95 / 117  191 / ..    577 / 650   (one wave per tile)
+//   16-bit C = 96     11 / 49    19 / 51    51 / 80   104 / 178  240 / 402  519 / ..   1300 / 2027  (one wave per tile)
+//   fp32 C = 16       10 / 14    10 / 14    14 / 15    20 / 23    39 / 52    75 / ..    166 / 206   (one wave per tile)
+//   fp32 C = 48       16 / 45    19 / 47    47 / 72    89 / 145  205 / 326  410 / ..    951 / 1533  (one wave per tile)
+//   fp32 C = 32       19 / 61    22 / 121   33 / 119   47 / 121   86 / 121  170 / 236   383 / 474
+//   fp32 C = 64       20 / 112   35 / 113   63 / 219  138 / 225  312 / 334  636 / 740  1472 / 1638
+// A staged block walks 512 (C = 128: 256) rows behind a barrier per tap or two, so small sets leave most CUs idle and
+// pay 27 taps' latency; a resident block takes 128 rows a step and no barrier, but every slice of output channels
+// gathers the rows again (2 slices at 16-bit C = 64, 8 at C = 128). 32 rows a wave from 96k rows and 64 from 600k at
+// C = 32 (77k rows: 17 / 18 / 29 us with 16 / 32 / 64; 184k: 34 / 25 / 30; 1M: 176 / 130 / 118).
+template <typename E, int C>
+static int launch_float(const ConvArgs& a, int64_t rows, int epilogue, hipStream_t s) {
+    if constexpr (sizeof(E) == 4 || C == 48 || C == 96) {
+        return launch_g2rf<E, C, 1>(a, epilogue, s);
+    } else if constexpr (C == 32) {
+        if (rows < 96 * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+        if (rows < 600 * 1024) return launch_g2rf<E, C, 2>(a, epilogue, s);
+        return launch_g2rf<E, C, 4>(a, epilogue, s);
+    } else {
+        if constexpr (C <= 128)
+            if (rows <= (C == 64 ? 128 : 32) * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+        return launch_g2f<E, C>(a, epilogue, s);
+    }
+}
+
+// Whether the resident or staged kernels take this convolution: Ci = Co of the widths of launch_float's table, 32-bit
+// buffer offsets and aligned vectors. Other widths (and 16-bit C = 16) run one wave per 16 rows, spconv_k.
 static bool g2f_fits(const ConvArgs& a, int Ci, int elt, int epilogue) {
     const int rb = Ci * elt;
-    return Ci == a.Co && Ci >= 32 && Ci % 16 == 0 &&
-           (rb == 64 || rb == 128 || rb == 256 || (elt == 2 && (rb == 512 || rb == 1024))) &&
+    const bool width = elt == 4 ? Ci == 16 || Ci == 32 || Ci == 48 || Ci == 64
+                                : Ci == 32 || Ci == 48 || Ci == 64 || Ci == 96 || Ci == 128 || Ci == 256 || Ci == 512;
+    return Ci == a.Co && width &&
            a.M * 27 * 4 < ((int64_t)1 << 31) && a.M * rb < ((int64_t)1 << 31) && aligned16(a.out) &&
            (epilogue != PMG_EPI_R || aligned16(a.skip));
 }
@@ -1074,11 +1166,13 @@ int launch_conv_f16_dev(const DevConv& d, hipStream_t s) {
     a.out = d.out;
     a.m_dev = d.m_dev;
     if (g2f_fits(a, d.Ci, 2, d.epilogue)) {
-        if (d.Ci == 32) return launch_g2f<_Float16, 32>(a, d.epilogue, s);
-        if (d.Ci == 64) return launch_g2f<_Float16, 64>(a, d.epilogue, s);
-        if (d.Ci == 128) return launch_g2f<_Float16, 128>(a, d.epilogue, s);
-        if (d.Ci == 256) return launch_g2f<_Float16, 256>(a, d.epilogue, s);
-        return launch_g2f<_Float16, 512>(a, d.epilogue, s);
+        if (d.Ci == 32) return launch_float<_Float16, 32>(a, d.expect, d.epilogue, s);
+        if (d.Ci == 48) return launch_float<_Float16, 48>(a, d.expect, d.epilogue, s);
+        if (d.Ci == 96) return launch_float<_Float16, 96>(a, d.expect, d.epilogue, s);
+        if (d.Ci == 64) return launch_float<_Float16, 64>(a, d.expect, d.epilogue, s);
+        if (d.Ci == 128) return launch_float<_Float16, 128>(a, d.expect, d.epilogue, s);
+        if (d.Ci == 256) return launch_float<_Float16, 256>(a, d.expect, d.epilogue, s);
+        return launch_float<_Float16, 512>(a, d.expect, d.epilogue, s);
     }
     return conv_common<_Float16>(a, d.Ci, d.epilogue, s);
 }
@@ -1172,11 +1266,13 @@ int pmg_spconv_f16(const uint16_t* x, const int32_t* nmap_t, const uint32_t* til
     ConvArgs a{(const uint8_t*)x, nmap_t, tile_mask, (const uint8_t*)w, M, Co, Ci * 2, Ci * 2 / 16,
                1.0f, nullptr, bias, 1.0f, skip, out};
     if (g2f_fits(a, Ci, 2, epilogue)) {
-        if (Ci == 32) return launch_g2f<_Float16, 32>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 64) return launch_g2f<_Float16, 64>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 128) return launch_g2f<_Float16, 128>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 256) return launch_g2f<_Float16, 256>(a, epilogue, (hipStream_t)stream);
-        return launch_g2f<_Float16, 512>(a, epilogue, (hipStream_t)stream);
+        if (Ci == 32) return launch_float<_Float16, 32>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 48) return launch_float<_Float16, 48>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 96) return launch_float<_Float16, 96>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 64) return launch_float<_Float16, 64>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 128) return launch_float<_Float16, 128>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 256) return launch_float<_Float16, 256>(a, a.M, epilogue, (hipStream_t)stream);
+        return launch_float<_Float16, 512>(a, a.M, epilogue, (hipStream_t)stream);
     }
     return conv_common<_Float16>(a, Ci, epilogue, (hipStream_t)stream);
 }
@@ -1191,11 +1287,13 @@ int pmg_spconv_bf16(const uint16_t* x, const int32_t* nmap_t, const uint32_t* ti
     ConvArgs a{(const uint8_t*)x, nmap_t, tile_mask, (const uint8_t*)w, M, Co, Ci * 2, Ci * 2 / 16,
                1.0f, nullptr, bias, 1.0f, skip, out};
     if (g2f_fits(a, Ci, 2, epilogue)) {
-        if (Ci == 32) return launch_g2f<__bf16, 32>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 64) return launch_g2f<__bf16, 64>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 128) return launch_g2f<__bf16, 128>(a, epilogue, (hipStream_t)stream);
-        if (Ci == 256) return launch_g2f<__bf16, 256>(a, epilogue, (hipStream_t)stream);
-        return launch_g2f<__bf16, 512>(a, epilogue, (hipStream_t)stream);
+        if (Ci == 32) return launch_float<__bf16, 32>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 48) return launch_float<__bf16, 48>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 96) return launch_float<__bf16, 96>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 64) return launch_float<__bf16, 64>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 128) return launch_float<__bf16, 128>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 256) return launch_float<__bf16, 256>(a, a.M, epilogue, (hipStream_t)stream);
+        return launch_float<__bf16, 512>(a, a.M, epilogue, (hipStream_t)stream);
     }
     return conv_common<__bf16>(a, Ci, epilogue, (hipStream_t)stream);
 }
@@ -1208,8 +1306,10 @@ int pmg_spconv_f32(const float* x, const int32_t* nmap_t, const uint32_t* tile_m
     ConvArgs a{(const uint8_t*)x, nmap_t, tile_mask, (const uint8_t*)w, M, Co, Ci * 4, Ci * 4 / 16,
                1.0f, nullptr, bias, 1.0f, nullptr, out};
     if (g2f_fits(a, Ci, 4, epilogue)) {
-        if (Ci == 32) return launch_g2f<float, 32>(a, epilogue, (hipStream_t)stream);
-        return launch_g2f<float, 64>(a, epilogue, (hipStream_t)stream);
+        if (Ci == 16) return launch_float<float, 16>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 32) return launch_float<float, 32>(a, a.M, epilogue, (hipStream_t)stream);
+        if (Ci == 48) return launch_float<float, 48>(a, a.M, epilogue, (hipStream_t)stream);
+        return launch_float<float, 64>(a, a.M, epilogue, (hipStream_t)stream);
     }
     return conv_common<float>(a, Ci, epilogue, (hipStream_t)stream);
 }

@@ -148,6 +148,7 @@ struct DevConv {
     void* out;
     int32_t* part;       // tap-split partial sums, or NULL
     int64_t part_bytes;
+    int64_t expect;      // the rows the level is expected to hold (a kernel's choice only; any count is computed)
 };
 int launch_conv_i8_dev(const DevConv& d, hipStream_t s);
 // The same for the fp16 teacher: x, w fp16 (the int8_t pointers hold fp16 data), fp32 accumulation, epilogues SILU

@@ -1330,6 +1330,7 @@ static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const 
     c1.tile_mask = u->tmask[k];
     c1.cap = u->cap;
     c1.m_dev = u->counts + k;
+    c1.expect = 2 * u->cap >> (2 * k);  // (A shape: 0.60, 0.16, 0.036, 0.0084 of the capacity at levels 1 to 4)
     c1.Ci = C;
     c1.Co = C;
     c1.w = (const int8_t*)bk.w1;

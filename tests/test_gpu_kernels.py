@@ -448,6 +448,47 @@ def test_conv_f32(gpu, Ci, Co):
     assert np.array_equal(got, acc + b)
 
 
+_FLOAT_CASES = [("f16", 32, m) for m in (1, 127, 98_303, 98_305, 614_401)] + [("bf16", 48, 129), ("f16", 48, 5_001)] + \
+    [("bf16", 64, m) for m in (2, 1_025, 131_072, 131_073)] + [("f16", 96, 3_000), ("bf16", 96, 17)] + \
+    [("f16", 128, m) for m in (15, 32_768, 32_769)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
+                                                                                 (48, 3_001), (64, 16), (64, 5_000))]
+
+
+@pytest.mark.parametrize("dtype,C,M", _FLOAT_CASES)
+def test_conv_float_dispatch(gpu, dtype, C, M):
+    """The float convolutions at the edges of their kernels' ranges (resident or staged weights by the row count, 16 to 64
+    rows a wave, rows that end inside a tile or a 64-byte chunk) on a random map with absent taps and rows without
+    any neighbour but themselves: the fp64 sums within the fp32-accumulation bound, and the bias and residual epilogues
+    on the kernel's own sums."""
+    announce(f"conv float dispatch {dtype} C={C} M={M}")
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dtype]
+    conv = {"f16": ops.spconv_f16, "bf16": ops.spconv_bf16}.get(dtype)
+    g = torch.Generator(device=gpu).manual_seed(C * 1000 + M)
+    rand = lambda *s: torch.randn(*s, generator=g, device=gpu)
+    nm = torch.randint(0, M, (M, 27), generator=g, device=gpu, dtype=torch.int32)
+    nm[torch.rand(M, 27, generator=g, device=gpu) < 0.7] = -1
+    nm[::5] = -1
+    nm[:, 13] = torch.arange(M, device=gpu, dtype=torch.int32)
+    nt, tm = ops.nmap_from_rows(nm)
+    x, w, b = rand(M, C).to(dt), (0.05 * rand(C, 3, 3, 3, C)).to(dt), rand(C)
+    got = conv(x, nt, tm, w) if conv else ops.spconv_f32(x, nt, tm, w)
+    xd, wd = x.double(), w.double().reshape(C, 27, C)
+    ref, mag = torch.zeros(M, C, dtype=torch.float64, device=gpu), torch.zeros(M, C, dtype=torch.float64, device=gpu)
+    for v in range(27):
+        rows = (nm[:, v] >= 0).nonzero()[:, 0]
+        src = nm[rows, v].long()
+        ref.index_add_(0, rows, xd[src] @ wd[:, v].T.contiguous())
+        mag.index_add_(0, rows, xd[src].abs() @ wd[:, v].abs().T.contiguous())
+    # fp32 accumulation of exact products (fp32: rounded ones): error bound ~ n_terms * eps32 * sum|terms|
+    assert ((got.double() - ref).abs() <= 27 * C * 2 ** -23 * mag + 1e-6).all()
+    if conv:
+        assert torch.equal(conv(x, nt, tm, w, ops.EPI_BIAS, bias=b), got + b)
+        skip = rand(M, C)
+        assert torch.equal(conv(x, nt, tm, w, ops.EPI_R, bias=b, skip=skip), (got + b) + skip)
+    else:
+        assert torch.equal(ops.spconv_f32(x, nt, tm, w, b), got + b)
+
+
 # ---------------------------------------------------------------------------------------------------------- row ops
 @pytest.mark.parametrize("C", [16, 32, 48, 64, 128])
 def test_ln_silu(gpu, C):
