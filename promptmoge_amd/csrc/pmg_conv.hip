@@ -344,6 +344,14 @@ __device__ inline void store_float4(const ConvArgs& a, int64_t o, const v4f& acc
 constexpr int kXcdGroup = 16;
 __host__ __device__ inline int xcd_group(int64_t nunits) { return nunits >= 8 * kXcdGroup ? kXcdGroup : 0; }
 
+// Blocks of a host-sized launch that walks nchunk chunks with at most `most` blocks: each XCD has a block for every
+// chunk that it is dealt, as far as they go. (A grid of nchunk blocks gave the later XCDs fewer blocks than chunks: int8
+// C = 128, 22 chunks of 512 rows: 101 us, whole rounds of 8 blocks 52; 157 chunks in groups: 104 and 55.)
+static int64_t walk_blocks(int64_t nchunk, int64_t most) {
+    const int64_t n = xcd_group(nchunk) ? most : (nchunk + 7) / 8 * 8;
+    return n < most ? n : most;
+}
+
 constexpr int kBufWord3 = 0x00020000;  // buffer descriptor word 3 for raw (untyped) loads on gfx9
 constexpr int kG2Threads = 512;       // 8 waves: two per SIMD, 256 registers each
 constexpr int kG2Waves = kG2Threads / 64;
@@ -887,7 +895,7 @@ static int launch_g2r(const ConvArgs& a, int epilogue, hipStream_t s) {
     if (cus < 0) cus = num_cus();
     constexpr int T = kG2rT, RS = kG2rRS, NWV = kG2rWaves, CHUNK = NWV * T * 16;
     const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
-    const dim3 grid((unsigned)(nchunk < cus ? nchunk : cus)), blk(64 * NWV);
+    const dim3 grid((unsigned)(walk_blocks(nchunk, cus))), blk(64 * NWV);
     switch (epilogue) {
         case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_ACC, T, 1, RS, NWV>), grid, blk, 0, s, a); break;
         case PMG_EPI_Q: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_Q, T, 1, RS, NWV>), grid, blk, 0, s, a); break;
@@ -911,7 +919,7 @@ static int launch_g2(const ConvArgs& a, int epilogue, hipStream_t s) {
         if (cus < 0) cus = num_cus();
         constexpr int T = kG2T128, RS = kG2RS128, CHUNK = kG2Waves * T * 16;
         const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
-        const dim3 grid((unsigned)(nchunk < cus ? nchunk : cus)), blk(kG2Threads);
+        const dim3 grid((unsigned)(walk_blocks(nchunk, cus))), blk(kG2Threads);
         switch (epilogue) {
             case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_ACC, C / 16, T, 1, RS, false>), grid, blk, 0, s, a); break;
             case PMG_EPI_Q: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_Q, C / 16, T, 1, RS, false>), grid, blk, 0, s, a); break;
@@ -937,7 +945,7 @@ static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
     constexpr int T = RB <= 128 ? 4 : (RB <= 512 ? 2 : 1), CHUNK = kG2Waves * T * 16;
     constexpr int PFV = RB >= 512 ? 4 : 1;  // weight operands read ahead (measured: 3 % faster at C = 256 / 512)
     const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
-    const dim3 grid((unsigned)(nchunk < cus ? nchunk : cus), (unsigned)(C / (16 * NB))), blk(kG2Threads);
+    const dim3 grid((unsigned)(walk_blocks(nchunk, cus)), (unsigned)(C / (16 * NB))), blk(kG2Threads);
     switch (epilogue) {
         case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_ACC, NB, T, PFV, 2, false, E>), grid, blk, 0, s, a); break;
         case PMG_EPI_BIAS: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_BIAS, NB, T, PFV, 2, false, E>), grid, blk, 0, s, a); break;
@@ -972,7 +980,7 @@ static int launch_g2rf(const ConvArgs& a, int epilogue, hipStream_t s) {
     int per = cus / (C / (16 * NB));
     if (per >= 8) per -= per % 8;
     const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
-    const dim3 grid((unsigned)(nchunk < per ? nchunk : per), (unsigned)(C / (16 * NB))), blk(kG2Threads);
+    const dim3 grid((unsigned)(walk_blocks(nchunk, per)), (unsigned)(C / (16 * NB))), blk(kG2Threads);
     switch (epilogue) {
         case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_ACC, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a); break;
         case PMG_EPI_BIAS: hipLaunchKernelGGL((spconv_g2r_k<C, PMG_EPI_BIAS, T, 1, 4, kG2Waves, E, NB>), grid, blk, 0, s, a); break;
@@ -995,20 +1003,20 @@ static int launch_g2rf(const ConvArgs& a, int epilogue, hipStream_t s) {
 
 // Ci = Co = C float features (g2f_fits): resident weights or staged ones, by the number of rows (a device-sized launch:
 // the rows its level is expected to hold). Measured on surface sets, one map, us, resident against staged:
-//   rows                2k         10k        30k        77k        184k       400k       1M
-//   16-bit C = 32     13 / 16    12 / 29    13 / 30    17 / 32    25 / 33    49 / 62    118 / 154
-//   16-bit C = 64     13 / 35    14 / 69    20 / 69    41 / 71    80 / 74   156 / 140   378 / 311
-//   16-bit C = 128    17 / 56    39 / 57    93 / 110  213 / 116   ..
-//   16-bit C = 48     11 / 20    11 / 21    21 / 26    40 / 54    95 / 117  191 / ..    577 / 650   (one wave per tile)
-//   16-bit C = 96     11 / 49    19 / 51    51 / 80   104 / 178  240 / 402  519 / ..   1300 / 2027  (one wave per tile)
-//   fp32 C = 16       10 / 14    10 / 14    14 / 15    20 / 23    39 / 52    75 / ..    166 / 206   (one wave per tile)
-//   fp32 C = 48       16 / 45    19 / 47    47 / 72    89 / 145  205 / 326  410 / ..    951 / 1533  (one wave per tile)
-//   fp32 C = 32       19 / 61    22 / 121   33 / 119   47 / 121   86 / 121  170 / 236   383 / 474
-//   fp32 C = 64       20 / 112   35 / 113   63 / 219  138 / 225  312 / 334  636 / 740  1472 / 1638
-// A staged block walks 512 (C = 128: 256) rows behind a barrier per tap or two, so small sets leave most CUs idle and
-// pay 27 taps' latency; a resident block takes 128 rows a step and no barrier, but every slice of output channels
+//   rows                2k         10k        30k        65k        77k        184k       400k       1M
+//   16-bit C = 32     11 / 16    11 / 16    11 / 17    11 / 17    17 / 18    25 / 33    50 / 63    118 / 151
+//   16-bit C = 64     12 / 35    12 / 36    20 / 37    34 / 39    40 / 39    81 / 74   156 / 140   379 / 310
+//   16-bit C = 128    17 / 56    39 / 56    91 / 59   172 / 62   212 / 113  488 / 172   ..
+//   16-bit C = 48     11 / 20    11 / 21    21 / 26    ..         40 / 54    95 / 117  191 / ..    577 / 650   (one wave per tile)
+//   16-bit C = 96     11 / 49    19 / 51    51 / 80    ..        104 / 178  240 / 402  519 / ..   1300 / 2027  (one wave per tile)
+//   fp32 C = 16       10 / 14    10 / 14    14 / 15    ..         20 / 23    39 / 52    75 / ..    166 / 206   (one wave per tile)
+//   fp32 C = 48       16 / 45    19 / 47    47 / 72    ..         89 / 145  205 / 326  410 / ..    951 / 1533  (one wave per tile)
+//   fp32 C = 32       19 / 61    20 / 61    20 / 61    37 / 62    52 / 64    87 / 123  170 / 235   383 / 475
+//   fp32 C = 64       20 / 112   36 / 112   65 / 113  118 / 118  142 / 222  315 / 332  638 / 741  1473 / 1645
+// A staged block walks 512 (C = 128: 256) rows behind a barrier per tap or two: one round of 256 blocks takes 27 taps'
+// time whatever the set. A resident block takes 128 rows a step and no barrier, but every slice of output channels
 // gathers the rows again (2 slices at 16-bit C = 64, 8 at C = 128). 32 rows a wave from 96k rows and 64 from 600k at
-// C = 32 (77k rows: 17 / 18 / 29 us with 16 / 32 / 64; 184k: 34 / 25 / 30; 1M: 176 / 130 / 118).
+// C = 32 (77k rows: 17 / 18 / 18 us with 16 / 32 / 64; 184k: 35 / 25 / 30; 1M: 180 / 131 / 118).
 template <typename E, int C>
 static int launch_float(const ConvArgs& a, int64_t rows, int epilogue, hipStream_t s) {
     if constexpr (sizeof(E) == 4 || C == 48 || C == 96) {
@@ -1019,7 +1027,7 @@ static int launch_float(const ConvArgs& a, int64_t rows, int epilogue, hipStream
         return launch_g2rf<E, C, 4>(a, epilogue, s);
     } else {
         if constexpr (C <= 128)
-            if (rows <= (C == 64 ? 128 : 32) * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+            if (rows <= (C == 64 ? 72 : 12) * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
         return launch_g2f<E, C>(a, epilogue, s);
     }
 }

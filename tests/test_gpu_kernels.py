@@ -449,8 +449,8 @@ def test_conv_f32(gpu, Ci, Co):
 
 
 _FLOAT_CASES = [("f16", 32, m) for m in (1, 127, 98_303, 98_305, 614_401)] + [("bf16", 48, 129), ("f16", 48, 5_001)] + \
-    [("bf16", 64, m) for m in (2, 1_025, 131_072, 131_073)] + [("f16", 96, 3_000), ("bf16", 96, 17)] + \
-    [("f16", 128, m) for m in (15, 32_768, 32_769)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
+    [("bf16", 64, m) for m in (2, 1_025, 73_728, 73_729, 131_073)] + [("f16", 96, 3_000), ("bf16", 96, 17)] + \
+    [("f16", 128, m) for m in (15, 12_288, 12_289, 32_769)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
                                                                                  (48, 3_001), (64, 16), (64, 5_000))]
 
 
