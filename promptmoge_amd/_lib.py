@@ -143,6 +143,7 @@ SIGNATURES = {
     "pmg_unet_workspace_bytes": (sz, [vp]),
     "pmg_unet_capacity": (i64, [vp]),
     "pmg_unet_set_weights": (i32, [vp, C.POINTER(UNetWeights)]),
+    "pmg_unet_set_fragments": (i32, [vp, C.POINTER(vp), i32]),
     "pmg_unet_forward": (i32, [vp, vp, vp, vp, vp, vp, vp, vp]),
     "pmg_unet_buffer": (vp, [vp, i32, i32]),
     "pmg_unet_step_prepare": (i32, [vp, C.POINTER(UNetStepConfig)]),

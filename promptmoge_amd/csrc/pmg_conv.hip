@@ -53,17 +53,48 @@ struct ConvArgs {
 // device: as many units as fit one round of blocks.
 constexpr int kSplitUnits = 256;  // units aimed at (chunks x output slices x Z): one block per CU of MI355X
 constexpr int kSplitMax = 9;
-__host__ __device__ inline int split_factor(int nchunk, int nslice) {
+__host__ __device__ inline int split_factor(int nchunk, int nslice, int units = kSplitUnits) {
     const int cs = nchunk * nslice;
-    const int z = cs > 0 ? kSplitUnits / cs : 1;
+    const int z = cs > 0 ? units / cs : 1;
     return z < 1 ? 1 : (z > kSplitMax ? kSplitMax : z);
 }
 
-// Row m, output channels c .. c+3 of a tap-split launch: the Z partial sums added in order (int32: exact, the
-// unsplit accumulator) and the epilogue of the device-sized convolution in the same arithmetic.
+// Epilogue of the float kernels: channels n .. n + 3 of one row (accumulators, their biases) at element o of the output.
 template <int EPI>
+__device__ inline void store_float4(const ConvArgs& a, int64_t o, const v4f& acc, const float* bias) {
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        y[i] = acc[i];
+        if constexpr (EPI != PMG_EPI_ACC) {
+            if (a.bias) y[i] = y[i] + bias[i];
+        }
+    }
+    if constexpr (EPI == PMG_EPI_SILU) {
+        float h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = silu_fast(y[i]);
+        store_half4(h, (_Float16*)a.out + o);
+    } else if constexpr (EPI == PMG_EPI_R) {
+        const v4f sk = *(const v4f*)(a.skip + o);
+        *(v4f*)((float*)a.out + o) = v4f{y[0] + sk[0], y[1] + sk[1], y[2] + sk[2], y[3] + sk[3]};
+    } else {
+        *(v4f*)((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
+    }
+}
+
+// Row m, output channels c .. c+3 of a tap-split launch: the Z partial sums added in order (int32: exact, the
+// unsplit accumulator; fp32 from the fp16 kernel) and the epilogue of the device-sized convolution in the same
+// arithmetic.
+template <int EPI, typename E>
 __device__ inline void split_finish(const ConvArgs& a, int Z, int M, int64_t m, int c) {
     const int Co = a.Co;
+    if constexpr (sizeof(E) != 1) {
+        v4f sum = *(const v4f*)((const float*)a.part + m * Co + c);
+        for (int z = 1; z < Z; ++z) sum += *(const v4f*)((const float*)a.part + ((int64_t)z * M + m) * Co + c);
+        store_float4<EPI>(a, m * Co + c, sum, a.bias + c);
+        return;
+    }
     v4i acc = *(const v4i*)(a.part + m * Co + c);
     for (int z = 1; z < Z; ++z) acc += *(const v4i*)(a.part + ((int64_t)z * M + m) * Co + c);
     const int64_t o = m * Co + c;
@@ -93,16 +124,16 @@ __device__ inline void split_finish(const ConvArgs& a, int Z, int M, int64_t m, 
 
 // The second launch of a tap split: the row count and Z read again on the device exactly as spconv_g2_k reads
 // them (CHUNK rows per chunk, nslice output slices); nothing to do when that launch did not split.
-template <int EPI, int CHUNK>
+template <int EPI, int CHUNK, typename E = int8_t, int UNITS = kSplitUnits>
 __global__ __launch_bounds__(256) void split_epilogue_k(ConvArgs a, int nslice) {
     const int M = (int)*a.m_dev;
-    const int Z = split_factor((M + CHUNK - 1) / CHUNK, nslice);
+    const int Z = split_factor((M + CHUNK - 1) / CHUNK, nslice, UNITS);
     if (Z < 2) return;
     const int Q4 = a.Co / 4;
     const int64_t total = (int64_t)M * Q4;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
         const int64_t m = e / Q4;
-        split_finish<EPI>(a, Z, M, m, 4 * (int)(e - m * Q4));
+        split_finish<EPI, E>(a, Z, M, m, 4 * (int)(e - m * Q4));
     }
 }
 
@@ -308,30 +339,6 @@ __device__ inline void store_tile_codes(const ConvArgs& a, const v4i (&acc)[T][N
                 *(v4i*)((int8_t*)a.out + (int64_t)orow[t] * Co + n0 + 64 * h + 16 * g) =
                     v4i{(int)q[0], (int)q[1], (int)q[2], (int)q[3]};
         }
-    }
-}
-
-// Epilogue of the float kernels: channels n .. n + 3 of one row (accumulators, their biases) at element o of the output.
-template <int EPI>
-__device__ inline void store_float4(const ConvArgs& a, int64_t o, const v4f& acc, const float* bias) {
-    float y[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        y[i] = acc[i];
-        if constexpr (EPI != PMG_EPI_ACC) {
-            if (a.bias) y[i] = y[i] + bias[i];
-        }
-    }
-    if constexpr (EPI == PMG_EPI_SILU) {
-        float h[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) h[i] = silu_fast(y[i]);
-        store_half4(h, (_Float16*)a.out + o);
-    } else if constexpr (EPI == PMG_EPI_R) {
-        const v4f sk = *(const v4f*)(a.skip + o);
-        *(v4f*)((float*)a.out + o) = v4f{y[0] + sk[0], y[1] + sk[1], y[2] + sk[2], y[3] + sk[3]};
-    } else {
-        *(v4f*)((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
     }
 }
 
@@ -886,6 +893,284 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Generic-map convolution with the gathered rows in LDS and the weights in registers, Ci = Co = C.
+//
+// A block of 4 waves owns 64 rows x BC output channels (64 at C = 64, else 128), each wave all 64 rows (4 tiles) x 16 NB
+// channels. Per step -- a tap of the chunk's union, or a 256-byte piece of its rows where they are longer -- the block
+// gathers its 64 neighbour rows once (each thread NP 16-byte pieces, two steps ahead, through registers into one of two
+// LDS buffers, a row's pieces permuted by the row so that operand reads meet no bank twice), and each wave loads its own
+// channels' weights from L2 straight into registers: up to 8 fragments two steps ahead. So a row is fetched once per
+// block, no weight passes through LDS, and a step has one barrier. Two blocks (C = 64: four) share a CU, so that one
+// block's loads and barriers run beside another's MFMAs; absent neighbours and rows past the end load zeros.
+//
+// The launch is bound by the weights' way into the registers: a wave-wide load of the plain [Co][27][Ci] layout touches
+// 16 rows of 64 bytes, one of the fragment order (PK: [Co / 16][27][row / 64 B][lane][16 B], laid out once by the
+// owner of the weights) 1 KB in one piece. Surface sets, us, the staged kernel / plain / fragment order:
+//   rows              2.6k              11k                49k               184k
+//   fp16 C = 64       35 / 13 / 15      36 / 13 / 15       37 / 29 / 22      74 / 97 / 62
+//   fp16 C = 128      56 / 31 / 26      57 / 32 / 27       62 / 87 / 59      -
+//   fp16 C = 256      75 / 56 / 42      78 / 108 / 62      298 / 312 / 184   -
+//   fp16 C = 512     102 / 107 / 90    289 / 309 / 199     -                 -
+//   int8 C = 128      52 / 19 / 19      52 / 19 / 19       54 / 47 / 41      109 / 162 / -
+//   int8 C = 256     103 / 39 / 33     186 / 71 / 50      599 / 180 / 115    -        (one wave per 16 rows for staged)
+// Tiles of 128 rows, waves of 128 x 32 or 64 x 64, and blocks of 8 waves were slower (C = 256, 11k rows, fragment order:
+// 62 - 90 us): they leave one block to a CU, or fewer waves than the loads' latency asks for.
+//
+// DEV: the row count is on the device. With partial sums (a.part) a level of few chunks splits the union's taps into Z
+// ranges (split_factor), added in order by split_epilogue_k. Output-channel slices go to groups of XCDs, so that a
+// slice's weights stay in the L2s that read them, and the chunks of a slice in bands to the XCDs of its group.
+constexpr int kTRows = 64, kTThreads = 256;
+constexpr int kTUnits = 512;  // blocks in flight: two per CU
+template <int C, typename E, int EPI, bool DEV, bool PK>
+__global__ __launch_bounds__(kTThreads, (C == 64 ? 4 : 2)) void spconv_t_k(ConvArgs a) {
+    constexpr int T = 4, NB = C == 64 ? 1 : 2, BC = 64 * NB, TH = kTThreads, BR = kTRows;
+    constexpr int RB = C * (int)sizeof(E), SB = RB < 256 ? RB : 256;  // row, and the part of it staged per step
+    constexpr int KS = SB / 64, SP = RB / SB;
+    constexpr int NSL = C / BC, XP = 8 / NSL;        // output-channel slices, XCDs per slice
+    constexpr int CH = SB / 16, NP = BR * CH / TH;   // 16-byte pieces per staged row, pieces per thread and step
+    constexpr int NF = KS * NB;                      // weight fragments per wave and step
+    static_assert(RB % SB == 0 && NP * TH == BR * CH && NF <= 8 && 8 % NSL == 0, "tile shape");
+    typedef typename Acc<E>::type acc_t;
+    typedef const __attribute__((address_space(3))) v4i lds_v4i;
+    __shared__ __attribute__((aligned(16))) v4i s_a[2][BR * CH];
+    __shared__ float s_k[2][BC];
+
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int S = (int)a.M;
+    const int M = DEV ? (int)*a.m_dev : S;
+    const int nchunk = (M + BR - 1) / BR;
+    const int Z = DEV && a.part ? split_factor(nchunk, NSL, kTUnits) : 1;
+    const int nunit = nchunk * Z;
+    const int xcd = blockIdx.x & 7, xb = xcd / NSL;  // (block b runs on XCD b % 8)
+    const int n0 = (xcd % NSL) * BC, nw = wv * 16 * NB;
+    const int u0 = (int)((int64_t)nunit * xb / XP), u1 = (int)((int64_t)nunit * (xb + 1) / XP);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, (int)(a.M * RB), kBufWord3);
+    const __amdgpu_buffer_rsrc_t nr =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.nmap_t, (short)0, (int)(a.M * 27 * 4), kBufWord3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, C * 27 * RB, kBufWord3);
+    constexpr int OOB = (int)0x80000000, END = 27 * SP;  // an out-of-range offset; the step past the last
+
+    for (int e = tid; e < 2 * BC; e += TH) {
+        const int q = e / BC, n = e - (e / BC) * BC;
+        const float* src = q == 0 ? a.w_scale : a.bias;
+        s_k[q][n] = src ? src[n0 + n] : 0.0f;
+    }
+    // the thread's pieces: row prow of the chunk, byte pofs of the staged part, LDS slot
+    int prow[NP], pofs[NP], pslot[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int id = tid + TH * p, row = id / CH, c = id - row * CH;
+        prow[p] = row;
+        pofs[p] = 16 * c;
+        pslot[p] = row * CH + (c ^ (row & 7));
+    }
+    const int wlane = PK ? 16 * lane + (n0 + nw) / 16 * (27 * 16 * RB) : (n0 + nw + r) * 27 * RB + 16 * g;
+
+    struct Cursor {
+        uint32_t rem;  // taps left
+        int h;         // next piece of the first of them
+    };
+    auto pop = [](Cursor& c) {  // the next step, tap * SP + piece, or END
+        const int v = c.rem ? (int)__builtin_ctz(c.rem) * SP + c.h : END;
+        const bool last = SP == 1 || c.h == SP - 1;
+        if (last) c.rem &= c.rem - 1;
+        c.h = last || v == END ? 0 : c.h + 1;
+        return v;
+    };
+
+    for (int un = u0 + (blockIdx.x >> 3); un < u1; un += gridDim.x >> 3) {
+        const int ch = Z == 1 ? un : un / Z, z = un - ch * Z;
+        uint32_t um;  // the taps of the chunk's rows
+        {
+            const int64_t ntile = (M + 15) >> 4, tl = (int64_t)ch * (BR / 16) + lane;
+            uint32_t u = lane < BR / 16 && tl < ntile ? a.tmask[tl] : 0u;
+            u |= __shfl_xor(u, 1, 64);
+            u |= __shfl_xor(u, 2, 64);
+            um = (uint32_t)__builtin_amdgcn_readfirstlane((int)u);
+        }
+        int nstep = __builtin_popcount(um) * SP;
+        if (DEV && Z > 1) {  // the z-th range of the taps
+            const int n = __builtin_popcount(um), k0 = n * z / Z, k1 = n * (z + 1) / Z;
+            for (int k = 0; k < k0; ++k) um &= um - 1;
+            uint32_t rest = um;
+            for (int k = k0; k < k1; ++k) rest &= rest - 1;
+            um ^= rest;
+            nstep = (k1 - k0) * SP;
+        }
+        int pcol[NP];  // the pieces' map columns
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const int pos = ch * BR + prow[p];
+            pcol[p] = pos < M ? 4 * pos : OOB;
+        }
+        auto idx_load = [&](int v, int (&id)[NP]) {
+            const int vo = v / SP * S * 4;  // (END: past the map)
+#pragma unroll
+            for (int p = 0; p < NP; ++p) id[p] = __builtin_amdgcn_raw_buffer_load_b32(nr, pcol[p], vo, 0);
+        };
+        auto gather = [&](int v, const int (&id)[NP], v4i (&x)[NP]) {
+            const int end = v < END ? 0 : OOB;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const int none = id[p] | pcol[p] | end;  // (one sign test: a branch here would drain all loads)
+                const int off = none < 0 ? OOB : id[p] * RB + pofs[p];
+                x[p] = __builtin_amdgcn_raw_buffer_load_b128(xr, off, SP == 1 ? 0 : v % SP * SB, 0);
+            }
+        };
+        auto w_load = [&](int v, int f) {  // fragment f = (K chunk f / NB, channel tile f % NB) of step v
+            const int s2 = f / NB, j = f - (f / NB) * NB;
+            const bool has = v < END;
+            const int tap = has ? v / SP : 0, k = (SP == 1 ? 0 : v % SP * KS) + s2;
+            const int so = PK ? ((j * 27 + tap) * (RB / 64) + k) * 1024 : (16 * j * 27 + tap) * RB + 64 * k;
+            return __builtin_amdgcn_raw_buffer_load_b128(wr, has ? wlane : OOB, so, 0);
+        };
+
+        acc_t acc[T][NB];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[t][j] = acc_t{0, 0, 0, 0};
+
+        Cursor ci{um, 0}, cg{um, 0}, cw{um, 0};  // map indices, gathers, weights
+        int I[2][NP];
+        v4i X[2][NP], W[2][NF];
+        {
+            int iu[2][NP];
+            idx_load(pop(ci), iu[0]);
+            idx_load(pop(ci), iu[1]);
+            idx_load(pop(ci), I[0]);
+            idx_load(pop(ci), I[1]);
+            gather(pop(cg), iu[0], X[0]);
+            gather(pop(cg), iu[1], X[1]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int v = pop(cw);
+#pragma unroll
+            for (int f = 0; f < NF; ++f) W[u][f] = w_load(v, f);
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) s_a[0][pslot[p]] = X[0][p];
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // (lgkmcnt(0): the loads in flight stay in flight)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+
+        auto step = [&](auto Kc) {
+            constexpr int K = decltype(Kc)::value;  // step number modulo 2
+            const int vw = pop(cw);
+            gather(pop(cg), I[K], X[K]);
+            idx_load(pop(ci), I[K]);
+            __builtin_amdgcn_sched_barrier(0);
+            const v4i* sa = s_a[K] + r * CH;
+            v4i A[2][T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) A[0][t] = *(lds_v4i*)(sa + t * 16 * CH + (g ^ (r & 7)));
+#pragma unroll
+            for (int s2 = 0; s2 < KS; ++s2) {
+                if (s2 + 1 < KS) {
+#pragma unroll
+                    for (int t = 0; t < T; ++t)
+                        A[(s2 + 1) & 1][t] = *(lds_v4i*)(sa + t * 16 * CH + ((4 * (s2 + 1) + g) ^ (r & 7)));
+                }
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const int f = s2 * NB + j;
+                    const v4i w = W[K][f];
+#pragma unroll
+                    for (int t = 0; t < T; ++t) mma(acc[t][j], w, A[s2 & 1][t], E{});
+                    W[K][f] = w_load(vw, f);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) s_a[K ^ 1][pslot[p]] = X[K ^ 1][p];
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll 1
+        for (int k = 0; k < nstep; k += 2) {  // (a step past the last multiplies zeros)
+            step(std::integral_constant<int, 0>{});
+            step(std::integral_constant<int, 1>{});
+        }
+
+        // lane (r, g) holds channels 16 j + 4 g .. + 3 of row r of each tile
+        int orow[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int p = ch * BR + 16 * t + r;
+            orow[t] = p < M ? (a.order ? a.order[p] : p) : -1;
+        }
+        if (DEV && Z > 1) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (orow[t] >= 0)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j)
+                        *(acc_t*)(a.part + ((int64_t)z * M + orow[t]) * C + n0 + nw + 16 * j + 4 * g) = acc[t][j];
+            continue;
+        }
+        if constexpr (sizeof(E) == 1 && (EPI == PMG_EPI_Q || EPI == PMG_EPI_QLIN)) {
+            static_assert(sizeof(E) != 1 || NB == 2, "code stores: two tiles of 32 channels at a time");
+#pragma unroll
+            for (int t = 0; t < T; t += 2) {
+                uint32_t q[4];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const int tt = t + h / 2, j = h & 1;
+                    float y[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int n = nw + 16 * j + 4 * g + i;
+                        float u = (float)acc[tt][j][i] * a.a_scale;
+                        u = u * s_k[0][n];
+                        if (a.bias) u = u + s_k[1][n];
+                        y[i] = u;
+                    }
+                    q[h] = EPI == PMG_EPI_Q ? pack_silu_codes4(y, a.out_mult) : pack_codes4(y, a.out_mult);
+                }
+                lane_groups_transpose4(q);  // lane group g: channels 16 (g & 1) .. + 15 of tile t + g / 2
+                const int row = g < 2 ? orow[t] : orow[t + 1];
+                if (row >= 0)
+                    *(v4i*)((int8_t*)a.out + (int64_t)row * C + n0 + nw + 16 * (g & 1)) =
+                        v4i{(int)q[0], (int)q[1], (int)q[2], (int)q[3]};
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (orow[t] < 0) continue;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const int n = nw + 16 * j + 4 * g;
+                    const int64_t o = (int64_t)orow[t] * C + n0 + n;
+                    if constexpr (sizeof(E) != 1) {
+                        store_float4<EPI>(a, o, acc[t][j], s_k[1] + n);
+                    } else if constexpr (EPI == PMG_EPI_ACC) {
+                        *(v4i*)((int32_t*)a.out + o) = acc[t][j];
+                    } else {
+                        float y[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float u = (float)acc[t][j][i] * a.a_scale;
+                            u = u * s_k[0][n + i];
+                            if (a.bias) u = u + s_k[1][n + i];
+                            y[i] = u;
+                        }
+                        if constexpr (EPI == PMG_EPI_R) {
+                            const v4f sk = *(const v4f*)(a.skip + o);
+                            *(v4f*)((float*)a.out + o) = v4f{y[0] + sk[0], y[1] + sk[1], y[2] + sk[2], y[3] + sk[3]};
+                        } else {
+                            *(v4f*)((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
+                        }
+                    }
+                }
+            }
+        }
+    }
+}
+
 // The host-sized C = 64 launch: 16-row tiles per wave, gather ring slots, waves per block.
 constexpr int kG2rT = 4, kG2rRS = 2, kG2rWaves = 8;
 
@@ -907,6 +1192,44 @@ static int launch_g2r(const ConvArgs& a, int epilogue, hipStream_t s) {
     return check_launch("spconv_g2r_k");
 }
 
+// The host-sized launch of spconv_t_k (plain weights).
+template <typename E, int C>
+static int launch_t(const ConvArgs& a, int epilogue, hipStream_t s) {
+    constexpr int XP = 8 / (C / (C == 64 ? 64 : 128));
+    const int64_t nchunk = (a.M + kTRows - 1) / kTRows;
+    const dim3 grid((unsigned)(8 * ((nchunk + XP - 1) / XP))), blk(kTThreads);
+    switch (epilogue) {
+        case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_ACC, false, false>), grid, blk, 0, s, a); break;
+        case PMG_EPI_BIAS: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_BIAS, false, false>), grid, blk, 0, s, a); break;
+        case PMG_EPI_R: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_R, false, false>), grid, blk, 0, s, a); break;
+        case PMG_EPI_Q:
+        case PMG_EPI_QLIN:
+            if constexpr (sizeof(E) == 1) {
+                if (epilogue == PMG_EPI_Q)
+                    hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_Q, false, false>), grid, blk, 0, s, a);
+                else
+                    hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_QLIN, false, false>), grid, blk, 0, s, a);
+                break;
+            }
+            [[fallthrough]];
+        case PMG_EPI_SILU:
+            if constexpr (std::is_same<E, _Float16>::value) {
+                if (epilogue == PMG_EPI_SILU) {
+                    hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_SILU, false, false>), grid, blk, 0, s, a);
+                    break;
+                }
+            }
+            [[fallthrough]];
+        default: return fail(PMG_E_INVALID, "spconv: epilogue not available for this precision");
+    }
+    return check_launch("spconv_t_k");
+}
+
+// int8 C = 128: up to this many rows the tile kernel, whose blocks walk 64 rows: 20 us for the staged kernel's 52 up to
+// 16k rows, 33 for 53 to 32k, 47 for 54 at 49k, 72 for 55 at 66k (a staged block walks 512 rows: 27 taps' time
+// whatever the set, up to 131k rows).
+constexpr int64_t kTileRows128 = 48 * 1024;
+
 // The host-sized C = 128 launch: 16-row tiles per wave and gather ring slots.
 constexpr int kG2T128 = 4, kG2RS128 = 2;
 
@@ -915,6 +1238,7 @@ static int launch_g2(const ConvArgs& a, int epilogue, hipStream_t s) {
     if constexpr (C == 64) {
         return launch_g2r<64>(a, epilogue, s);
     } else {
+        if (a.M <= kTileRows128) return launch_t<int8_t, 128>(a, epilogue, s);
         static int cus = -1;
         if (cus < 0) cus = num_cus();
         constexpr int T = kG2T128, RS = kG2RS128, CHUNK = kG2Waves * T * 16;
@@ -959,6 +1283,37 @@ static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
         default: return fail(PMG_E_INVALID, "spconv: epilogue not available for this precision");
     }
     return check_launch("spconv_g2_k");
+}
+
+// The device-sized fp16 launch on fragment-ordered weights: blocks for twice the rows expected (more rows: each block
+// walks its band), the tap split when the partials buffer holds its largest case (Z * rows * C * 4 bytes, Z * chunks *
+// slices <= kTUnits), followed by split_epilogue_k.
+template <int C>
+static int launch_t_dev(const ConvArgs& a, int64_t expect, int epilogue, hipStream_t s) {
+    constexpr int NSL = C / (C == 64 ? 64 : 128), XP = 8 / NSL;
+    int64_t nchunk = (a.M + kTRows - 1) / kTRows;
+    const int64_t want = (2 * expect + kTRows - 1) / kTRows, least = kTUnits / NSL;
+    if (nchunk > want) nchunk = want;
+    if (nchunk < least) nchunk = least;  // (the tap split's units, too)
+    const dim3 grid((unsigned)(8 * ((nchunk + XP - 1) / XP))), blk(kTThreads);
+    typedef _Float16 E;
+    switch (epilogue) {
+        case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_ACC, true, true>), grid, blk, 0, s, a); break;
+        case PMG_EPI_SILU: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_SILU, true, true>), grid, blk, 0, s, a); break;
+        case PMG_EPI_R: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_R, true, true>), grid, blk, 0, s, a); break;
+        default: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_BIAS, true, true>), grid, blk, 0, s, a); break;
+    }
+    if (int e = check_launch("spconv_t_k")) return e;
+    if (!a.part) return PMG_OK;
+    const int64_t blocks = (a.M * (C / 4) + 255) / 256;
+    const dim3 egrid((unsigned)(blocks < 1024 ? blocks : 1024));
+    switch (epilogue) {
+        case PMG_EPI_ACC: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_ACC, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
+        case PMG_EPI_SILU: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_SILU, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
+        case PMG_EPI_R: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_R, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
+        default: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_BIAS, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
+    }
+    return check_launch("split_epilogue_k");
 }
 
 // Float features on resident weights (spconv_g2r_k): the slice of output channels whose 27 taps fit the LDS (108 KB at
@@ -1016,7 +1371,9 @@ static int launch_g2rf(const ConvArgs& a, int epilogue, hipStream_t s) {
 // A staged block walks 512 (C = 128: 256) rows behind a barrier per tap or two: one round of 256 blocks takes 27 taps'
 // time whatever the set. A resident block takes 128 rows a step and no barrier, but every slice of output channels
 // gathers the rows again (2 slices at 16-bit C = 64, 8 at C = 128). 32 rows a wave from 96k rows and 64 from 600k at
-// C = 32 (77k rows: 17 / 18 / 18 us with 16 / 32 / 64; 184k: 35 / 25 / 30; 1M: 180 / 131 / 118).
+// C = 32 (77k rows: 17 / 18 / 18 us with 16 / 32 / 64; 184k: 35 / 25 / 30; 1M: 180 / 131 / 118). In between the tile
+// kernel (spconv_t_k) on the plain weights: C = 128 31 us up to 16k rows, one round of its blocks (resident 39 at 11k, 50
+// at 15k; staged 57; two rounds 58), C = 256 56 up to 8k (staged 75), 108 beyond (78).
 template <typename E, int C>
 static int launch_float(const ConvArgs& a, int64_t rows, int epilogue, hipStream_t s) {
     if constexpr (sizeof(E) == 4 || C == 48 || C == 96) {
@@ -1026,8 +1383,16 @@ static int launch_float(const ConvArgs& a, int64_t rows, int epilogue, hipStream
         if (rows < 600 * 1024) return launch_g2rf<E, C, 2>(a, epilogue, s);
         return launch_g2rf<E, C, 4>(a, epilogue, s);
     } else {
-        if constexpr (C <= 128)
-            if (rows <= (C == 64 ? 72 : 12) * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+        if constexpr (C == 64) {
+            if (rows <= 72 * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+        }
+        if constexpr (C == 128) {
+            if (rows <= (a.m_dev ? 12 : 8) * 1024) return launch_g2rf<E, C, 1>(a, epilogue, s);
+            if (!a.m_dev && rows <= 16 * 1024) return launch_t<E, C>(a, epilogue, s);
+        }
+        if constexpr (C == 256) {
+            if (!a.m_dev && rows <= 8 * 1024) return launch_t<E, C>(a, epilogue, s);
+        }
         return launch_g2f<E, C>(a, epilogue, s);
     }
 }
@@ -1098,7 +1463,8 @@ static int launch_g2_dev_split(ConvArgs a, int epilogue, int32_t* part, int64_t 
     return check_launch("split_epilogue_k");
 }
 
-int64_t conv_split_bytes(int C) {
+int64_t conv_split_bytes(int C, bool f16) {
+    if (f16) return C == 128 || C == 256 || C == 512 ? (int64_t)kTUnits * kTRows * 128 * 4 : 0;
     if (C == 128) return (int64_t)kSplitUnits * (kG2Waves * 2 * 16) * 128 * 4;
     if (C == 256) return (int64_t)kSplitUnits * (kG2Waves * 1 * 16) * 128 * 4;
     return 0;
@@ -1174,6 +1540,14 @@ int launch_conv_f16_dev(const DevConv& d, hipStream_t s) {
     a.out = d.out;
     a.m_dev = d.m_dev;
     if (g2f_fits(a, d.Ci, 2, d.epilogue)) {
+        if (d.wf && (d.Ci == 64 || d.Ci == 128 || d.Ci == 256 || d.Ci == 512)) {
+            a.w = (const uint8_t*)d.wf;
+            a.part = d.part && d.part_bytes > 0 && d.part_bytes >= conv_split_bytes(d.Ci, true) ? d.part : nullptr;
+            if (d.Ci == 64) return launch_t_dev<64>(a, d.expect, d.epilogue, s);
+            if (d.Ci == 128) return launch_t_dev<128>(a, d.expect, d.epilogue, s);
+            if (d.Ci == 256) return launch_t_dev<256>(a, d.expect, d.epilogue, s);
+            return launch_t_dev<512>(a, d.expect, d.epilogue, s);
+        }
         if (d.Ci == 32) return launch_float<_Float16, 32>(a, d.expect, d.epilogue, s);
         if (d.Ci == 48) return launch_float<_Float16, 48>(a, d.expect, d.epilogue, s);
         if (d.Ci == 96) return launch_float<_Float16, 96>(a, d.expect, d.epilogue, s);
@@ -1237,10 +1611,11 @@ int pmg_spconv_i8(const int8_t* x, const int32_t* nmap_t, const uint32_t* tile_m
                a_scale, w_scale, bias, out_mult, skip, out};
     // The block-tiled kernel addresses x and the map through 32-bit buffer offsets.
     const bool fits32 = M * 27 * 4 < ((int64_t)1 << 31) && M * Ci < ((int64_t)1 << 31);
-    if (Ci == Co && (Ci == 64 || Ci == 128) && fits32 && epilogue != PMG_EPI_SILU && aligned16(out) &&
+    if (Ci == Co && (Ci == 64 || Ci == 128 || Ci == 256) && fits32 && epilogue != PMG_EPI_SILU && aligned16(out) &&
         aligned16(x) && aligned16(w) && (epilogue != PMG_EPI_R || aligned16(skip))) {
         if (Ci == 64) return launch_g2<64>(a, epilogue, (hipStream_t)stream);
-        return launch_g2<128>(a, epilogue, (hipStream_t)stream);
+        if (Ci == 128) return launch_g2<128>(a, epilogue, (hipStream_t)stream);
+        return launch_t<int8_t, 256>(a, epilogue, (hipStream_t)stream);
     }
     return conv_common<int8_t>(a, Ci, epilogue, (hipStream_t)stream);
 }

@@ -1180,6 +1180,13 @@ using namespace pmg;
 
 // ---------------------------------------------------------------------------------------------------------------
 // The U-Net context: one arena holding every level's structure and activations at the level-0 capacity.
+// A residual block's weights, and its convolutions' in fragment order (NULL: none given).
+struct UnetBlock : pmg_block_weights {
+    const void* f1 = nullptr;
+    const void* f2 = nullptr;
+    UnetBlock(const pmg_block_weights& b) : pmg_block_weights(b) {}
+};
+
 struct pmg_unet {
     pmg_unet_config cfg{};
     int L = 0;
@@ -1234,7 +1241,7 @@ struct pmg_unet {
     const float* pr_b = nullptr;
     const float* out_w = nullptr;
     const float* out_b = nullptr;
-    std::vector<pmg_block_weights> down[kMaxLevels], dec[kMaxLevels], bott;
+    std::vector<UnetBlock> down[kMaxLevels], dec[kMaxLevels], bott;
     std::vector<pmg_linear_weights> pool, up;
     pmg_linear_weights enc{}, fuse0{}, fuse2{};
 
@@ -1266,7 +1273,7 @@ struct UnetOut {
 // One residual block on level k (flex_sparse_blocks.py:70-75) whose conv1 input codes are in u->q1 and whose stream
 // is x (updated in place). After conv2: the next block's LayerNorm codes (level 0: fused RLN epilogue; else the row
 // kernel), nothing, or (last level-0 block of the network) out_proj into `rout`.
-static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const pmg_block_weights* next, float* x,
+static int enqueue_block(pmg_unet* u, int k, const UnetBlock& bk, const UnetBlock* next, float* x,
                          const UnetOut* rout, hipStream_t s) {
     const int C = u->cfg.channels[k];
     const bool f16 = u->cfg.precision == PMG_PREC_FP16;
@@ -1334,6 +1341,7 @@ static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const 
     c1.Ci = C;
     c1.Co = C;
     c1.w = (const int8_t*)bk.w1;
+    c1.wf = bk.f1;
     c1.epilogue = f16 ? PMG_EPI_SILU : PMG_EPI_Q;
     c1.a_scale = bk.a1_scale;
     c1.w_scale = bk.w1_scale;
@@ -1342,7 +1350,7 @@ static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const 
     c1.out = u->q2;
     // the tap split (a second launch) only at the coarsest level: the capacity does not bound a level's rows, and
     // at the finer levels, with too many rows to split, that launch would only cost its dispatch
-    if (k == u->L - 1 && k > 0 && !f16) {
+    if (k == u->L - 1) {
         c1.part = u->part;
         c1.part_bytes = u->part_bytes;
     }
@@ -1351,6 +1359,7 @@ static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const 
     DevConv c2 = c1;
     c2.x = (const int8_t*)u->q2;
     c2.w = (const int8_t*)bk.w2;
+    c2.wf = bk.f2;
     c2.epilogue = PMG_EPI_R;
     c2.a_scale = bk.a2_scale;
     c2.w_scale = bk.w2_scale;
@@ -1365,10 +1374,10 @@ static int enqueue_block(pmg_unet* u, int k, const pmg_block_weights& bk, const 
 }
 
 // A stage of blocks on level k over stream x, whose first block's input codes are already in q1.
-static int enqueue_stage(pmg_unet* u, int k, const std::vector<pmg_block_weights>& st, float* x, const UnetOut* rout,
+static int enqueue_stage(pmg_unet* u, int k, const std::vector<UnetBlock>& st, float* x, const UnetOut* rout,
                          hipStream_t s) {
     for (size_t j = 0; j < st.size(); ++j) {
-        const pmg_block_weights* next = j + 1 < st.size() ? &st[j + 1] : nullptr;
+        const UnetBlock* next = j + 1 < st.size() ? &st[j + 1] : nullptr;
         if (int e = enqueue_block(u, k, st[j], next, x, next ? nullptr : rout, s)) return e;
     }
     return PMG_OK;
@@ -1779,7 +1788,7 @@ pmg_unet* pmg_unet_create(const pmg_unet_config* cfg) {
     take((void**)&u->lin, (size_t)4 * cap * u->Cmax);
     take((void**)&u->enc_codes, elt * u->T * c.enc_channels);
     take((void**)&u->enc_tok, (size_t)4 * u->T * CL);
-    if (L > 1 && c.precision != PMG_PREC_FP16) u->part_bytes = conv_split_bytes(c.channels[L - 1]);
+    if (L > 1) u->part_bytes = conv_split_bytes(c.channels[L - 1], c.precision == PMG_PREC_FP16);
     if (u->part_bytes > 0) take((void**)&u->part, (size_t)u->part_bytes);
     for (auto& p : plan) off += ualign(p.second);
     u->arena_bytes = off;
@@ -1879,6 +1888,23 @@ int pmg_unet_set_weights(pmg_unet* u, const pmg_unet_weights* w) {
     u->fuse2 = w->linears[L + 1];
     u->up.assign(w->linears + L + 2, w->linears + 2 * L + 1);
     u->have_weights = true;
+    u->graphs.clear();
+    return PMG_OK;
+}
+
+int pmg_unet_set_fragments(pmg_unet* u, const void* const* frag, int n) {
+    PMG_REQUIRE(u && frag, "null argument");
+    PMG_REQUIRE(u->have_weights, "set the weights first");
+    PMG_REQUIRE(u->cfg.precision == PMG_PREC_FP16, "fragment-ordered weights are fp16");
+    std::vector<UnetBlock*> blocks;
+    for (int k = 0; k < u->L; ++k)
+        for (UnetBlock& b : u->down[k]) blocks.push_back(&b);
+    for (UnetBlock& b : u->bott) blocks.push_back(&b);
+    for (int i = 0; i + 1 < u->L; ++i)
+        for (UnetBlock& b : u->dec[i]) blocks.push_back(&b);
+    PMG_REQUIRE(n == 2 * (int)blocks.size(), "fragment count mismatch: expected " + std::to_string(2 * blocks.size()));
+    for (int i = 0; i < n; ++i) PMG_REQUIRE(aligned16(frag[i]), "fragment-ordered weights must be 16-byte aligned");
+    for (int i = 0; i < n; ++i) (i % 2 ? blocks[i / 2]->f2 : blocks[i / 2]->f1) = frag[i];
     u->graphs.clear();
     return PMG_OK;
 }

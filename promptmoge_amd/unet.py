@@ -65,6 +65,7 @@ class UNetDeviceWeights:
                 dev(b.gamma), dev(b.beta), dev(q1, torch.int8), dev(s1), dev(b.b1), float(act_scale(b.clip1)),
                 float(act_mult(b.clip1)), dev(q2, torch.int8), dev(s2), dev(b.b2), float(act_scale(b.clip2)),
                 float(act_mult(b.clip2)))
+        self.fragments = self._fragment_order(w, len(blocks)) if f16 else None
         linears = list(w.pool) + [w.enc, w.fuse0, w.fuse2] + list(w.up)
         self._linears = (LinearWeights * len(linears))()
         for k, l in enumerate(linears):
@@ -77,6 +78,32 @@ class UNetDeviceWeights:
         self.struct = UNetWeights(self.in_w, self.in_b, self.pr_w, self.pr_b, self.out_w, self.out_b, len(blocks),
                                   C.cast(self._blocks, C.POINTER(BlockWeights)), len(linears),
                                   C.cast(self._linears, C.POINTER(LinearWeights)))
+
+    def _fragment_order(self, w: UNetW, n: int):
+        """The conv weights of the levels >= 1 that have them, in one buffer in the order of pmg_unet_set_fragments."""
+        levels = [k for k, st in enumerate(w.down) for _ in st] + [w.levels - 1] * len(w.bott) + \
+                 [w.levels - 2 - i for i, st in enumerate(w.dec) for _ in st]
+        plain = {x.data_ptr(): x for x in self.keep}
+        want = [(2 * k + j, plain[p]) for k in range(n) if levels[k] > 0 and w.channels[levels[k]] in (64, 128, 256, 512)
+                for j, p in enumerate((self._blocks[k].w1, self._blocks[k].w2))]
+        frag = (_lib.vp * (2 * n))()
+        if want:
+            flat = torch.empty(sum(x.numel() for _, x in want), dtype=torch.float16, device=want[0][1].device)
+            self.keep.append(flat)
+            at = 0
+            for q, x in want:  # element (n, tap, k) at [n / 16][tap][k / 32][k % 32 / 8][n % 16][k % 8]
+                co, ci = x.shape[0], x.shape[-1]
+                y = flat[at:at + x.numel()]
+                y.view(co // 16, 27, ci // 32, 4, 16, 8).copy_(x.view(co // 16, 16, 27, ci // 32, 4, 8).permute(0, 2, 3, 4, 1, 5))
+                frag[q] = y.data_ptr()
+                at += x.numel()
+        return frag
+
+    def give(self, h) -> None:
+        """Sets these weights in a context (pmg_unet_create)."""
+        call("pmg_unet_set_weights", h, C.byref(self.struct))
+        if self.fragments is not None:
+            call("pmg_unet_set_fragments", h, self.fragments, len(self.fragments))
 
 
 class UNetRefiner(torch.nn.Module):
@@ -145,7 +172,7 @@ class UNetRefiner(torch.nn.Module):
             h = lib().pmg_unet_create(C.byref(cfg))
             if not h:
                 raise _lib.PmgError(_lib.PMG_E_INVALID, lib().pmg_last_error().decode())
-            call("pmg_unet_set_weights", h, C.byref(dw.struct))
+            dw.give(h)
             self._ctx[key] = h
             M = B * H * W
             w = self.host_weights
@@ -303,7 +330,7 @@ class UNetStep:
             self.h = lib().pmg_unet_create(C.byref(cfg))
             if not self.h:
                 raise _lib.PmgError(_lib.PMG_E_INVALID, lib().pmg_last_error().decode())
-            call("pmg_unet_set_weights", self.h, C.byref(self.weights.struct))
+            self.weights.give(self.h)
             scfg = UNetStepConfig(self.dh, self.dw, int(fit_iters), float(fit_trim), int(fit_min_points),
                                   int(use_prompt), int(soft_gate), int(output_gate), float(output_gate_floor),
                                   float(anchor), int(final_fit))

@@ -450,7 +450,7 @@ def test_conv_f32(gpu, Ci, Co):
 
 _FLOAT_CASES = [("f16", 32, m) for m in (1, 127, 98_303, 98_305, 614_401)] + [("bf16", 48, 129), ("f16", 48, 5_001)] + \
     [("bf16", 64, m) for m in (2, 1_025, 73_728, 73_729, 131_073)] + [("f16", 96, 3_000), ("bf16", 96, 17)] + \
-    [("f16", 128, m) for m in (15, 12_288, 12_289, 32_769)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
+    [("f16", 128, m) for m in (15, 8_192, 8_193, 16_384, 16_385)] + [("bf16", 128, 8_200), ("f16", 256, 1), ("f16", 256, 65), ("bf16", 256, 8_192), ("f16", 256, 8_193)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
                                                                                  (48, 3_001), (64, 16), (64, 5_000))]
 
 
@@ -487,6 +487,32 @@ def test_conv_float_dispatch(gpu, dtype, C, M):
         assert torch.equal(conv(x, nt, tm, w, ops.EPI_R, bias=b, skip=skip), (got + b) + skip)
     else:
         assert torch.equal(ops.spconv_f32(x, nt, tm, w, b), got + b)
+
+
+@pytest.mark.parametrize("C,M", [(128, 1), (128, 63), (128, 65), (128, 8_193), (128, 49_152), (128, 49_153), (256, 15),
+                                 (256, 64), (256, 5_001)])
+def test_conv_int8_tiles(gpu, C, M):
+    """int8 C = 128 and 256 at the edges of the tile kernel's chunks and of its range, on a random map with absent taps:
+    every epilogue bit for bit that of one wave per 16 rows, which takes outputs that are not 16-byte aligned."""
+    announce(f"conv int8 tiles C={C} M={M}")
+    g = torch.Generator(device=gpu).manual_seed(C + M)
+    nm = torch.randint(0, M, (M, 27), generator=g, device=gpu, dtype=torch.int32)
+    nm[torch.rand(M, 27, generator=g, device=gpu) < 0.7] = -1
+    nm[::5] = -1
+    nm[:, 13] = torch.arange(M, device=gpu, dtype=torch.int32)
+    nt, tm = ops.nmap_from_rows(nm)
+    codes = lambda *s: torch.randint(-127, 128, s, generator=g, device=gpu, dtype=torch.int8)
+    x, w = codes(M, C), codes(C, 3, 3, 3, C)
+    sc, b, skip = (torch.rand(C, generator=g, device=gpu) * 1e-3, torch.randn(C, generator=g, device=gpu),
+                   torch.randn(M, C, generator=g, device=gpu))
+    for epi, dt, kw in ((ops.EPI_ACC, torch.int32, {}), (ops.EPI_BIAS, torch.float32, {}), (ops.EPI_R, torch.float32, {"skip": skip}),
+                        (ops.EPI_Q, torch.int8, {"out_mult": 9.5}), (ops.EPI_QLIN, torch.int8, {"out_mult": 9.5})):
+        if epi != ops.EPI_ACC:
+            kw = {"a_scale": 0.02, "w_scale": sc, "bias": b, **kw}
+        off = 4 if dt == torch.int8 else 1
+        ref = torch.empty(M * C + off, dtype=dt, device=gpu)[off:].view(M, C)
+        ops.spconv_i8(x, nt, tm, w, epi, out=ref, **kw)
+        assert torch.equal(ops.spconv_i8(x, nt, tm, w, epi, **kw), ref), epi
 
 
 # ---------------------------------------------------------------------------------------------------------- row ops

@@ -5,6 +5,8 @@ masks too), the stream after every stage, the encoder tokens and the (M, 1) outp
 log depth (coords None) equals the one with _voxelize's coords; graph replays repeat the first result. The oracle's
 composition is pinned against the reference's own Sparse3DUNet (tests/test_oracle_unet.py).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -13,6 +15,7 @@ from oracle import structure as ost
 from oracle import unet as ou
 from promptmoge_amd import spec
 from promptmoge_amd import unet_weights as uw
+from promptmoge_amd._lib import call
 from promptmoge_amd.unet import UNetRefiner
 
 from conftest import announce
@@ -187,6 +190,36 @@ F16_CASES = {
 
 def _rms(a):
     return float(np.sqrt(np.mean(np.square(np.asarray(a, np.float64)))))
+
+
+@pytest.mark.parametrize("channels,B,H,W,noise", [((32, 64, 128, 256, 512), 1, 64, 96, 0.0), ((16, 128, 512, 64), 2, 40, 56, 0.0),
+                                                  ((16, 64, 256, 128), 1, 128, 160, 0.6)])
+def test_unet_fp16_fragments(gpu, channels, B, H, W, noise):
+    """Convolutions on fragment-ordered weights (tap split at the coarsest level, levels with more rows than their
+    blocks were launched for: depth noise keeps most voxels apart) against the same module on the plain ones, whose
+    kernels take taps and channels in the same order: the same output but for the tap split's partial sums (a coarsest
+    width of 128 and more), within three times the 1e-3 RMS by which a different fp32 summation order moves it."""
+    announce(f"unet fp16 fragments {channels} {B}x{H}x{W}")
+    L = len(channels)
+    ds = 2 ** (L - 1)
+    w = uw.make_unet_weights(channels, 32, enc_blocks=[1] * L, dec_blocks=[1] * (L - 1), bottleneck_blocks=1, seed=5)
+    cfg = spec.StepConfig("u", H, W, 0.9 * W, 0.9 * W, W / 2, H / 2, channels[0], 1, "int8", seed=5)
+    pts = np.stack([spec.make_scene(cfg, seed=b).points for b in range(B)])
+    rng = np.random.default_rng(5)
+    pts[..., 2] += noise * rng.normal(size=pts.shape[:3]).astype(np.float32)
+    enc = _t(rng.normal(0, 1, (B, 32, H // ds, W // ds)).astype(np.float32), gpu)
+    _, coords, zext, _ = ost.voxelize(pts)
+    shape = torch.Size([B, H, W, zext, 3])
+    mod = UNetRefiner(w, precision="fp16")
+    tf = _t(pts.reshape(-1, 3), gpu)
+    out = mod(tf, None, shape, enc).double().cpu()
+    counts = mod.buffer("counts", 0).cpu().numpy()
+    assert not noise or counts[2] > 4 * (B * H * W >> 4)
+    for key, h in mod._ctx.items():
+        call("pmg_unet_set_weights", h, C.byref(mod._weights[key[0]].struct))
+    plain = mod(tf, None, shape, enc).double().cpu()
+    assert channels[-1] >= 128 or torch.equal(out, plain)
+    assert float((out - plain).square().mean().sqrt()) < 3e-3 * float(plain.square().mean().sqrt())
 
 
 @pytest.mark.parametrize("name", list(F16_CASES))
