@@ -19,7 +19,8 @@
 // Layers (int8 contract qat.py:1-16; the deployed engine's sequence, Refiner.swift:224-292, Refiner.metal:133-322):
 //   level-0 blocks         the map-free column convolutions (pmg_conv_col.hip) with the next LayerNorm fused
 //   blocks at levels >= 1  generic-map MFMA conv with the device row count (launch_conv_i8_dev: the weight-staged
-//                          spconv_g2_k / spconv_g2r_k at C = 64 / 128 / 256, spconv_k otherwise) + a row
+//                          spconv_g2_k / spconv_g2r_k at C = 64 / 128 / 256, spconv_k otherwise; fp16: the tile kernel
+//                          spconv_t_k at C = 64 to 512 on fragment-ordered weights) + a row
 //                          LayerNorm kernel
 //   PoolDown               one kernel: children's fp32 mean (row order, / count) quantised, int8 GEMM, and the next
 //                          block's LayerNorm codes (fp16: mean-pool kernel, GEMM, row LayerNorm kernel)
