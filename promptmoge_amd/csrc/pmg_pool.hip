@@ -6,15 +6,18 @@
 // the distinct parent keys in increasing order (torch.unique(sorted=True)); `parent` maps every input voxel to
 // its output row; `seg_indices` is the stable argsort of `parent` (the input rows grouped by output row, each
 // group in input order) and `seg_offsets` the group boundaries. All of it comes from one stable LSD radix sort of
-// (key, input row) pairs over the key's significant bits (8 bits per pass, three kernels per pass as below),
+// (key, input row) pairs over the key's significant bits (8 bits per pass, two to five kernels per pass as below),
 // after which a flag marks each first occurrence of a key and an exclusive scan of the flags numbers the
 // output rows. The number of output rows is written to device memory (the caller reads it once, as the
 // reference's int(...) does).
 //
-// Radix pass, over tiles of 2048 keys: pool_hist_k counts the tile's digits (LDS atomics), pool_scan_k (one
-// block) turns the digit-major counts into each (digit, tile)'s output base, pool_scatter_k places the keys of
-// each tile in 8 rounds of 256: a key's rank among equal digits of its round comes from 9 wave ballots plus the
-// counts of the lower waves, so the pass is stable and deterministic.
+// Radix pass, over tiles of 2048 keys: pool_hist_k counts the tile's digits (LDS atomics), a scan turns the counts
+// into each (digit, tile)'s output base, pool_scatter_k places the keys of each tile in 8 rounds of 256: a key's
+// rank among equal digits of its round comes from 9 wave ballots plus the counts of the lower waves, so the pass is
+// stable and deterministic. Up to kDirectTiles tiles every scatter block makes its own bases from all tiles' counts
+// instead (a pass is two launches, not four or five: each launch is 2 - 4 us of device time and about as much of the
+// caller's: a row order of 77k rows, three passes, 106 -> 66 us; 260k rows 116 -> 94); the scan's launches win where a
+// block would read hundreds of counts per digit.
 //
 // sparse_pool: one thread per (output row, 4 channels) sums its group's rows in seg_indices order -- input order,
 // the order of the reference's index_add_ -- in fp32 and divides by the group size ('mean'). sparse_upsample:
@@ -29,6 +32,7 @@ namespace pmg {
 constexpr int kPoolThreads = 256;
 constexpr int kPoolRounds = 8;
 constexpr int kPoolTile = kPoolThreads * kPoolRounds;  // 2048 keys per tile
+constexpr int kDirectTiles = 128;
 
 struct PoolGeom {
     int64_t in[4];   // B, X, Y, Z of the input grid
@@ -65,7 +69,8 @@ __global__ __launch_bounds__(kPoolThreads) void pool_hist_k(const uint64_t* __re
         if (i < M) atomicAdd(&h[(keys[i] >> shift) & 0xffu], 1u);
     }
     __syncthreads();
-    hist[(int64_t)threadIdx.x * ntile + blockIdx.x] = h[threadIdx.x];
+    hist[ntile <= kDirectTiles ? (int64_t)blockIdx.x * 256 + threadIdx.x  // (tile-major: read whole by each block)
+                               : (int64_t)threadIdx.x * ntile + blockIdx.x] = h[threadIdx.x];
 }
 
 // One block of 1024 threads: exclusive scan of n counts in place; the total goes to *total if given.
@@ -200,14 +205,40 @@ __global__ __launch_bounds__(kPoolThreads) void pool_scatter_k(const uint64_t* _
     __shared__ uint32_t run[256];      // keys of each digit this tile has placed
     __shared__ uint32_t cnt[NW][256];  // this round's count of each digit per wave
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    run[tid] = off[(int64_t)tid * ntile + blockIdx.x];
     const uint64_t below = (1ull << lane) - 1ull;
     const int64_t base = (int64_t)blockIdx.x * kPoolTile;
+    // every round's pairs are requested at once: a round's barriers then wait for no memory
+    uint64_t keys[kPoolRounds];
+    int32_t vals[kPoolRounds];
+#pragma unroll
     for (int k = 0; k < kPoolRounds; ++k) {
         const int64_t i = base + k * kPoolThreads + tid;
-        const bool ok = i < M;
-        const uint64_t key = ok ? keys_in[i] : 0ull;
-        const int32_t val = ok ? (vals_in ? vals_in[i] : (int32_t)i) : 0;
+        keys[k] = i < M ? keys_in[i] : 0ull;
+        vals[k] = i < M ? (vals_in ? vals_in[i] : (int32_t)i) : 0;
+    }
+    if (ntile <= kDirectTiles) {
+        // digit tid: its keys in the tiles before this one, and all keys of smaller digits
+        uint32_t before = 0, all = 0;
+#pragma unroll 16
+        for (int t = 0; t < ntile; ++t) {
+            const uint32_t c = off[t * 256 + tid];
+            all += c;
+            before += t < (int)blockIdx.x ? c : 0u;
+        }
+        const uint32_t inc = wave_incl_scan_u32(all);
+        if (lane == 63) cnt[0][w] = inc;
+        __syncthreads();
+        for (int q = 0; q < w; ++q) before += cnt[0][q];
+        run[tid] = before + inc - all;
+        __syncthreads();
+    } else {
+        run[tid] = off[(int64_t)tid * ntile + blockIdx.x];
+    }
+#pragma unroll
+    for (int k = 0; k < kPoolRounds; ++k) {
+        const bool ok = base + k * kPoolThreads + tid < M;
+        const uint64_t key = keys[k];
+        const int32_t val = vals[k];
         const uint32_t d = ok ? (uint32_t)((key >> shift) & 0xffu) : 256u;  // 256 matches no real digit
         uint64_t peers = __ballot(ok);
 #pragma unroll
@@ -391,7 +422,8 @@ int radix_sort_pairs(RadixBufs& r, int64_t M, int bits, int32_t* vals_final, hip
         int32_t* vout = pass == npass - 1 ? vals_final : r.vals[cur ^ 1];
         hipLaunchKernelGGL(pool_hist_k, dim3(nt), dim3(kPoolThreads), 0, s, kin, M, shift, nt, r.hist);
         if (int e = check_launch("pool_hist_k")) return e;
-        if (int e = pool_scan(r.hist, 256 * nt, nullptr, r.ctot, s)) return e;
+        if (nt > kDirectTiles)
+            if (int e = pool_scan(r.hist, 256 * nt, nullptr, r.ctot, s)) return e;
         hipLaunchKernelGGL(pool_scatter_k, dim3(nt), dim3(kPoolThreads), 0, s, kin, vin, M, shift, nt,
                            (const uint32_t*)r.hist, kout, vout);
         if (int e = check_launch("pool_scatter_k")) return e;
