@@ -1257,9 +1257,10 @@ static int launch_g2(const ConvArgs& a, int epilogue, hipStream_t s) {
 }
 
 // fp16 / bf16 features, Ci = Co = C with rows of 128 - 1024 bytes: the weight-staged kernel on K chunks of 32 halves
-// (v_mfma_f32_16x16x32_f16 / _bf16), fp32 accumulators. Rows of 256 bytes hold 16 tiles of accumulators per wave at T = 4, so they run T = 2; rows of 512 and 1024 bytes (fp16
-// C = 256, 512) split the output channels into slices of 64 (blockIdx.y: a tap's weights fit the LDS buffers) and
-// run T = 2 and 1 (the gathered rows of the two ring slots fill the registers).
+// (v_mfma_f32_16x16x32_f16 / _bf16), fp32 accumulators. Rows of 256 bytes hold 16 tiles of accumulators per wave at
+// T = 4, so they run T = 2; rows of 512 and 1024 bytes (fp16 C = 256, 512) split the output channels into slices of 64
+// (blockIdx.y: a tap's weights fit the LDS buffers) and run T = 2 and 1 (the gathered rows of the two ring slots fill
+// the registers).
 template <typename E, int C>
 static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
     static int cus = -1;
@@ -1514,9 +1515,9 @@ template <typename T>
 static int conv_common(const ConvArgs& a, int Ci, int epilogue, hipStream_t s);
 
 // The fp16 teacher's convolution on a device-sized level (the int8 one's counterpart): x and w fp16, fp32
-// accumulation; epilogues SILU (bias, SiLU, fp16 out: conv1), R (bias + skip, fp32: conv2), BIAS, ACC. The
-// weight-staged kernel takes Ci = Co = 32, 64, 128 (it reads the row count on the device); other widths the generic
-// one-wave-per-16-rows kernel.
+// accumulation; epilogues SILU (bias, SiLU, fp16 out: conv1), R (bias + skip, fp32: conv2), BIAS, ACC. The tile kernel
+// where the weights are there in fragment order (C = 64 - 512), else resident or staged weights by the rows expected
+// (launch_float; all read the row count on the device); other widths the generic one-wave-per-16-rows kernel.
 int launch_conv_f16_dev(const DevConv& d, hipStream_t s) {
     PMG_REQUIRE(d.x && d.nmap_t && d.tile_mask && d.w && d.out && d.m_dev, "null buffer");
     PMG_REQUIRE(d.Ci % 16 == 0 && d.Co % 16 == 0 && d.Ci > 0 && d.Co > 0, "channels must be multiples of 16");
