@@ -16,8 +16,11 @@
 // rank among equal digits of its round comes from 9 wave ballots plus the counts of the lower waves, so the pass is
 // stable and deterministic. Up to kDirectTiles tiles every scatter block makes its own bases from all tiles' counts
 // instead (a pass is two launches, not four or five: each launch is 2 - 4 us of device time and about as much of the
-// caller's: a row order of 77k rows, three passes, 106 -> 66 us; 260k rows 116 -> 94); the scan's launches win where a
-// block would read hundreds of counts per digit.
+// caller's: a row order of 77k rows, three passes, 106 -> 66 us); the scan's launches win where a block would read hundreds
+// of counts per digit. Row order and pool cache by the number of keys, us, scan / bases by each block:
+//   keys        268k        307k        420k        512k        648k        762k        900k        1040k
+//   row order   103 / 76    104 / 80    108 / 94    109 / 96    116 / 110   120 / 114   132 / 133   143 / 153
+//   pool cache  136 / 112   135 / 112   139 / 127   140 / 128   174 / 164   177 / 167   187 / 184   197 / 206
 //
 // sparse_pool: one thread per (output row, 4 channels) sums its group's rows in seg_indices order -- input order,
 // the order of the reference's index_add_ -- in fp32 and divides by the group size ('mean'). sparse_upsample:
@@ -32,7 +35,7 @@ namespace pmg {
 constexpr int kPoolThreads = 256;
 constexpr int kPoolRounds = 8;
 constexpr int kPoolTile = kPoolThreads * kPoolRounds;  // 2048 keys per tile
-constexpr int kDirectTiles = 128;
+constexpr int kDirectTiles = 384;
 
 struct PoolGeom {
     int64_t in[4];   // B, X, Y, Z of the input grid

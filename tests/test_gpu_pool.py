@@ -44,13 +44,15 @@ def test_pool_cache_matches_oracle(gpu, n, B, ext, stride):
     _check_cache(coords, (B, *ext), stride, gpu)
 
 
-@pytest.mark.parametrize("n", [2_047, 2_049, 262_144, 262_145])
-def test_pool_cache_at_the_radix_paths_edges(gpu, n):
-    """One tile of 2048 keys and two, and the most tiles whose counts the scatter blocks add up themselves and one more."""
+@pytest.mark.parametrize("n,ext", [(2_047, (100, 90, 80)), (2_049, (100, 90, 80)), (262_144, (100, 90, 80)),
+                                   (262_145, (100, 90, 80)), (786_432, (200, 180, 160)), (786_433, (200, 180, 160))])
+def test_pool_cache_at_the_radix_paths_edges(gpu, n, ext):
+    """One tile of 2048 keys and two, 128 and one more, and the most tiles whose counts the scatter blocks add up
+    themselves and one more."""
     announce(f"pool cache n={n}")
-    coords = _coords(np.random.default_rng(n), n + n // 4, 1, (100, 90, 80))[:n]
+    coords = _coords(np.random.default_rng(n), n + n // 4, 1, ext)[:n]
     assert len(coords) == n
-    _check_cache(coords, (1, 100, 90, 80), (2, 2, 2), gpu)
+    _check_cache(coords, (1, *ext), (2, 2, 2), gpu)
 
 
 def test_pool_cache_level0_raster(gpu):
