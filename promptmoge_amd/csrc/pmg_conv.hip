@@ -53,9 +53,9 @@ struct ConvArgs {
 // device: as many units as fit one round of blocks.
 constexpr int kSplitUnits = 256;  // units aimed at (chunks x output slices x Z): one block per CU of MI355X
 constexpr int kSplitMax = 9;
-__host__ __device__ inline int split_factor(int nchunk, int nslice, int units = kSplitUnits) {
+__host__ __device__ inline int split_factor(int nchunk, int nslice) {
     const int cs = nchunk * nslice;
-    const int z = cs > 0 ? units / cs : 1;
+    const int z = cs > 0 ? kSplitUnits / cs : 1;
     return z < 1 ? 1 : (z > kSplitMax ? kSplitMax : z);
 }
 
@@ -84,17 +84,10 @@ __device__ inline void store_float4(const ConvArgs& a, int64_t o, const v4f& acc
 }
 
 // Row m, output channels c .. c+3 of a tap-split launch: the Z partial sums added in order (int32: exact, the
-// unsplit accumulator; fp32 from the fp16 kernel) and the epilogue of the device-sized convolution in the same
-// arithmetic.
-template <int EPI, typename E>
+// unsplit accumulator) and the epilogue of the device-sized convolution in the same arithmetic.
+template <int EPI>
 __device__ inline void split_finish(const ConvArgs& a, int Z, int M, int64_t m, int c) {
     const int Co = a.Co;
-    if constexpr (sizeof(E) != 1) {
-        v4f sum = *(const v4f*)((const float*)a.part + m * Co + c);
-        for (int z = 1; z < Z; ++z) sum += *(const v4f*)((const float*)a.part + ((int64_t)z * M + m) * Co + c);
-        store_float4<EPI>(a, m * Co + c, sum, a.bias + c);
-        return;
-    }
     v4i acc = *(const v4i*)(a.part + m * Co + c);
     for (int z = 1; z < Z; ++z) acc += *(const v4i*)(a.part + ((int64_t)z * M + m) * Co + c);
     const int64_t o = m * Co + c;
@@ -124,16 +117,16 @@ __device__ inline void split_finish(const ConvArgs& a, int Z, int M, int64_t m, 
 
 // The second launch of a tap split: the row count and Z read again on the device exactly as spconv_g2_k reads
 // them (CHUNK rows per chunk, nslice output slices); nothing to do when that launch did not split.
-template <int EPI, int CHUNK, typename E = int8_t, int UNITS = kSplitUnits>
+template <int EPI, int CHUNK>
 __global__ __launch_bounds__(256) void split_epilogue_k(ConvArgs a, int nslice) {
     const int M = (int)*a.m_dev;
-    const int Z = split_factor((M + CHUNK - 1) / CHUNK, nslice, UNITS);
+    const int Z = split_factor((M + CHUNK - 1) / CHUNK, nslice);
     if (Z < 2) return;
     const int Q4 = a.Co / 4;
     const int64_t total = (int64_t)M * Q4;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
         const int64_t m = e / Q4;
-        split_finish<EPI, E>(a, Z, M, m, 4 * (int)(e - m * Q4));
+        split_finish<EPI>(a, Z, M, m, 4 * (int)(e - m * Q4));
     }
 }
 
@@ -917,9 +910,10 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
 // Tiles of 128 rows, waves of 128 x 32 or 64 x 64, and blocks of 8 waves were slower (C = 256, 11k rows, fragment order:
 // 62 - 90 us): they leave one block to a CU, or fewer waves than the loads' latency asks for.
 //
-// DEV: the row count is on the device. With partial sums (a.part) a level of few chunks splits the union's taps into Z
-// ranges (split_factor), added in order by split_epilogue_k. Output-channel slices go to groups of XCDs, so that a
-// slice's weights stay in the L2s that read them, and the chunks of a slice in bands to the XCDs of its group.
+// DEV: the row count is on the device. Output-channel slices go to groups of XCDs, so that a slice's weights stay in the
+// L2s that read them, and the chunks of a slice in bands to the XCDs of its group. Taps and channels are summed in
+// ascending order in one accumulator, as by the staged and resident kernels: the same bits. (No tap split: fp32 partial
+// sums of tap ranges would add up in another order.)
 constexpr int kTRows = 64, kTThreads = 256;
 constexpr int kTUnits = 512;  // blocks in flight: two per CU
 template <int C, typename E, int EPI, bool DEV, bool PK>
@@ -941,11 +935,9 @@ __global__ __launch_bounds__(kTThreads, (C == 64 ? 4 : 2)) void spconv_t_k(ConvA
     const int S = (int)a.M;
     const int M = DEV ? (int)*a.m_dev : S;
     const int nchunk = (M + BR - 1) / BR;
-    const int Z = DEV && a.part ? split_factor(nchunk, NSL, kTUnits) : 1;
-    const int nunit = nchunk * Z;
     const int xcd = blockIdx.x & 7, xb = xcd / NSL;  // (block b runs on XCD b % 8)
     const int n0 = (xcd % NSL) * BC, nw = wv * 16 * NB;
-    const int u0 = (int)((int64_t)nunit * xb / XP), u1 = (int)((int64_t)nunit * (xb + 1) / XP);
+    const int u0 = (int)((int64_t)nchunk * xb / XP), u1 = (int)((int64_t)nchunk * (xb + 1) / XP);
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, (int)(a.M * RB), kBufWord3);
     const __amdgpu_buffer_rsrc_t nr =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.nmap_t, (short)0, (int)(a.M * 27 * 4), kBufWord3);
@@ -980,8 +972,7 @@ __global__ __launch_bounds__(kTThreads, (C == 64 ? 4 : 2)) void spconv_t_k(ConvA
         return v;
     };
 
-    for (int un = u0 + (blockIdx.x >> 3); un < u1; un += gridDim.x >> 3) {
-        const int ch = Z == 1 ? un : un / Z, z = un - ch * Z;
+    for (int ch = u0 + (blockIdx.x >> 3); ch < u1; ch += gridDim.x >> 3) {
         uint32_t um;  // the taps of the chunk's rows
         {
             const int64_t ntile = (M + 15) >> 4, tl = (int64_t)ch * (BR / 16) + lane;
@@ -990,15 +981,7 @@ __global__ __launch_bounds__(kTThreads, (C == 64 ? 4 : 2)) void spconv_t_k(ConvA
             u |= __shfl_xor(u, 2, 64);
             um = (uint32_t)__builtin_amdgcn_readfirstlane((int)u);
         }
-        int nstep = __builtin_popcount(um) * SP;
-        if (DEV && Z > 1) {  // the z-th range of the taps
-            const int n = __builtin_popcount(um), k0 = n * z / Z, k1 = n * (z + 1) / Z;
-            for (int k = 0; k < k0; ++k) um &= um - 1;
-            uint32_t rest = um;
-            for (int k = k0; k < k1; ++k) rest &= rest - 1;
-            um ^= rest;
-            nstep = (k1 - k0) * SP;
-        }
+        const int nstep = __builtin_popcount(um) * SP;
         int pcol[NP];  // the pieces' map columns
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -1102,15 +1085,6 @@ __global__ __launch_bounds__(kTThreads, (C == 64 ? 4 : 2)) void spconv_t_k(ConvA
         for (int t = 0; t < T; ++t) {
             const int p = ch * BR + 16 * t + r;
             orow[t] = p < M ? (a.order ? a.order[p] : p) : -1;
-        }
-        if (DEV && Z > 1) {
-#pragma unroll
-            for (int t = 0; t < T; ++t)
-                if (orow[t] >= 0)
-#pragma unroll
-                    for (int j = 0; j < NB; ++j)
-                        *(acc_t*)(a.part + ((int64_t)z * M + orow[t]) * C + n0 + nw + 16 * j + 4 * g) = acc[t][j];
-            continue;
         }
         if constexpr (sizeof(E) == 1 && (EPI == PMG_EPI_Q || EPI == PMG_EPI_QLIN)) {
             static_assert(sizeof(E) != 1 || NB == 2, "code stores: two tiles of 32 channels at a time");
@@ -1287,15 +1261,14 @@ static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
 }
 
 // The device-sized fp16 launch on fragment-ordered weights: blocks for twice the rows expected (more rows: each block
-// walks its band), the tap split when the partials buffer holds its largest case (Z * rows * C * 4 bytes, Z * chunks *
-// slices <= kTUnits), followed by split_epilogue_k.
+// walks its band).
 template <int C>
 static int launch_t_dev(const ConvArgs& a, int64_t expect, int epilogue, hipStream_t s) {
     constexpr int NSL = C / (C == 64 ? 64 : 128), XP = 8 / NSL;
     int64_t nchunk = (a.M + kTRows - 1) / kTRows;
     const int64_t want = (2 * expect + kTRows - 1) / kTRows, least = kTUnits / NSL;
     if (nchunk > want) nchunk = want;
-    if (nchunk < least) nchunk = least;  // (the tap split's units, too)
+    if (nchunk < least) nchunk = least;
     const dim3 grid((unsigned)(8 * ((nchunk + XP - 1) / XP))), blk(kTThreads);
     typedef _Float16 E;
     switch (epilogue) {
@@ -1304,17 +1277,7 @@ static int launch_t_dev(const ConvArgs& a, int64_t expect, int epilogue, hipStre
         case PMG_EPI_R: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_R, true, true>), grid, blk, 0, s, a); break;
         default: hipLaunchKernelGGL((spconv_t_k<C, E, PMG_EPI_BIAS, true, true>), grid, blk, 0, s, a); break;
     }
-    if (int e = check_launch("spconv_t_k")) return e;
-    if (!a.part) return PMG_OK;
-    const int64_t blocks = (a.M * (C / 4) + 255) / 256;
-    const dim3 egrid((unsigned)(blocks < 1024 ? blocks : 1024));
-    switch (epilogue) {
-        case PMG_EPI_ACC: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_ACC, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
-        case PMG_EPI_SILU: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_SILU, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
-        case PMG_EPI_R: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_R, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
-        default: hipLaunchKernelGGL((split_epilogue_k<PMG_EPI_BIAS, kTRows, E, kTUnits>), egrid, dim3(256), 0, s, a, NSL); break;
-    }
-    return check_launch("split_epilogue_k");
+    return check_launch("spconv_t_k");
 }
 
 // Float features on resident weights (spconv_g2r_k): the slice of output channels whose 27 taps fit the LDS (108 KB at
@@ -1464,8 +1427,7 @@ static int launch_g2_dev_split(ConvArgs a, int epilogue, int32_t* part, int64_t 
     return check_launch("split_epilogue_k");
 }
 
-int64_t conv_split_bytes(int C, bool f16) {
-    if (f16) return C == 128 || C == 256 || C == 512 ? (int64_t)kTUnits * kTRows * 128 * 4 : 0;
+int64_t conv_split_bytes(int C) {
     if (C == 128) return (int64_t)kSplitUnits * (kG2Waves * 2 * 16) * 128 * 4;
     if (C == 256) return (int64_t)kSplitUnits * (kG2Waves * 1 * 16) * 128 * 4;
     return 0;
@@ -1543,7 +1505,6 @@ int launch_conv_f16_dev(const DevConv& d, hipStream_t s) {
     if (g2f_fits(a, d.Ci, 2, d.epilogue)) {
         if (d.wf && (d.Ci == 64 || d.Ci == 128 || d.Ci == 256 || d.Ci == 512)) {
             a.w = (const uint8_t*)d.wf;
-            a.part = d.part && d.part_bytes > 0 && d.part_bytes >= conv_split_bytes(d.Ci, true) ? d.part : nullptr;
             if (d.Ci == 64) return launch_t_dev<64>(a, d.expect, d.epilogue, s);
             if (d.Ci == 128) return launch_t_dev<128>(a, d.expect, d.epilogue, s);
             if (d.Ci == 256) return launch_t_dev<256>(a, d.expect, d.epilogue, s);

@@ -1351,7 +1351,7 @@ static int enqueue_block(pmg_unet* u, int k, const UnetBlock& bk, const UnetBloc
     c1.out = u->q2;
     // the tap split (a second launch) only at the coarsest level: the capacity does not bound a level's rows, and
     // at the finer levels, with too many rows to split, that launch would only cost its dispatch
-    if (k == u->L - 1) {
+    if (k == u->L - 1 && !f16) {
         c1.part = u->part;
         c1.part_bytes = u->part_bytes;
     }
@@ -1789,7 +1789,7 @@ pmg_unet* pmg_unet_create(const pmg_unet_config* cfg) {
     take((void**)&u->lin, (size_t)4 * cap * u->Cmax);
     take((void**)&u->enc_codes, elt * u->T * c.enc_channels);
     take((void**)&u->enc_tok, (size_t)4 * u->T * CL);
-    if (L > 1) u->part_bytes = conv_split_bytes(c.channels[L - 1], c.precision == PMG_PREC_FP16);
+    if (L > 1 && c.precision != PMG_PREC_FP16) u->part_bytes = conv_split_bytes(c.channels[L - 1]);
     if (u->part_bytes > 0) take((void**)&u->part, (size_t)u->part_bytes);
     for (auto& p : plan) off += ualign(p.second);
     u->arena_bytes = off;
