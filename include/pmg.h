@@ -283,6 +283,11 @@ unsigned pmg_debug_fit_spin_limit(unsigned polls);
  * finite residual (the radix passes follow its miss); 3: windows of 2^21-key bins (split passes); 0 (or any other
  * value) restores the normal plan. Results do not depend on the plan. Returns the previous mode. ABI version 5. */
 unsigned pmg_debug_fit_plan(unsigned mode);
+/* Test hook (no counterpart in the reference; no GPU needed): where a fit of N elements keeps the elements that its blocks
+ * exchange in a selection stage of the given parity. out[0] = blocks, out[1] = elements per block; byte offsets in the
+ * workspace of out[2] keys, out[3] z, out[4] targets (4 bytes an element, block after block) and out[5] pairs of z and
+ * target (8 bytes an element). */
+int pmg_debug_fit_exchange(int64_t N, int iters, int parity, int64_t* out);
 int pmg_fit_scale_shift(const float* z, const float* target, const uint8_t* mask, int B, int64_t N, int iters,
                         float trim, int min_points, float* st, int32_t* info, void* workspace,
                         size_t workspace_bytes, void* stream);

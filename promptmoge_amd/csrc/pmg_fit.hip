@@ -80,10 +80,21 @@ struct FitWs {
     unsigned* err_seen;   // launches whose bounded wait expired since the owner last cleared it (sticky)
     uint64_t* partials;   // [2][kFitMaxBlocks][5] fp64 bit patterns
     unsigned* hist;       // [iters][kFitHistSlots][kFitHistWords]
-    uint32_t* c_key;      // [2][nb][elements per block]: residual bits | mask << 31
-    float* c_z;           // [2][nb][elements per block]
-    float* c_t;           // [2][nb][elements per block]
+    uint32_t* exch;       // elements exchanged by a stage, by its parity (FitExchange)
 };
+
+// Where the elements that a stage exchanges lie, in words from FitWs::exch, for launches of `cap` = nb x elements per
+// block elements: key (residual bits | mask << 31), z and target of a bracket stage's candidates, [nb][elements per
+// block] each, or the (z, target) pairs of a local stage's uncertain elements, [nb][elements per block][2]. A block may
+// write stage n + 1's while a slower one still reads stage n's (fit_barrier), so the two parities share no word:
+// a parity's z and targets, and its pairs, take the same 2 cap words.
+struct FitExchange {
+    int64_t key, z, t, pairs;
+};
+__host__ __device__ constexpr FitExchange fit_exchange(int64_t cap, int parity) {
+    const int64_t zt = 2 * cap + parity * 2 * cap;
+    return {parity * cap, zt, zt + cap, zt};
+}
 
 struct FitArgs {
     int mode;  // 0: (z, target, mask) arrays; 1: prompt map (logz, LiDAR, conf); 2: final fit, LiDAR at the map's size
@@ -787,8 +798,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         v[0] = (double)nm;
         unsigned nub;
         unsigned slot = block_excl_scan((unsigned)__popc(unc), sh.tmp, nub);
-        // the pairs (z, target) take the memory of a stage's c_z and c_t together: one 8-byte load per element
-        float2* const pairs = (float2*)ws.c_z + (size_t)(stage & 1) * cap_words;
+        // pairs (z, target): one 8-byte load per element
+        float2* const pairs = (float2*)(ws.exch + fit_exchange(cap_words, stage & 1).pairs);
         {
             const size_t base = (size_t)b * kFitPerBlock;
 #pragma unroll
@@ -1159,16 +1170,20 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             const unsigned packed = block_excl_scan(((unsigned)below << 16) | (unsigned)nc, sh.tmp, packed_total);
             unsigned slot = packed & 0xffffu;
             const unsigned ncb = packed_total & 0xffffu;
-            const size_t base = (size_t)(stage & 1) * cap_words + (size_t)b * kFitPerBlock;
+            const FitExchange ex = fit_exchange(cap_words, stage & 1);
+            const size_t base = (size_t)b * kFitPerBlock;
+            uint32_t* const c_key = ws.exch + ex.key;
+            float* const c_z = (float*)(ws.exch + ex.z);
+            float* const c_t = (float*)(ws.exch + ex.t);
 #pragma unroll
             for (int g = 0; g < kFitEPT; g += 4) {
                 if (__any((cm >> g) & 15u)) {  // few elements are candidates: most waves skip most groups
 #pragma unroll
                     for (int j = g; j < g + 4; ++j) {
                         if ((cm >> j) & 1u) {
-                            ws.c_key[base + slot] = rb[j] | (((mbits >> j) & 1u) << 31);
-                            ws.c_z[base + slot] = zr[j];
-                            ws.c_t[base + slot] = tr[j];
+                            c_key[base + slot] = rb[j] | (((mbits >> j) & 1u) << 31);
+                            c_z[base + slot] = zr[j];
+                            c_t[base + slot] = tr[j];
                             ++slot;
                         }
                     }
@@ -1209,7 +1224,10 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         auto select_and_solve = [&](uint32_t blo, uint32_t bhi) {
             const unsigned total = sh.total_cand;
             unsigned rank = kk - sh.total_below;
-            const size_t bufo = (size_t)(stage & 1) * cap_words;
+            const FitExchange ex = fit_exchange(cap_words, stage & 1);
+            const uint32_t* const c_key = ws.exch + ex.key;
+            const float* const c_z = (const float*)(ws.exch + ex.z);
+            const float* const c_t = (const float*)(ws.exch + ex.t);
             // Thread (r, j) = (tid % nb, tid / nb) owns slots j, j + per, j + 2 per, ... of block r's region: no
             // search from a flat index to a region, and its loads are independent. Keys go to LDS in flat order
             // (region r at off[r]); the first kHold of the thread's candidates also keep z and target in registers
@@ -1220,7 +1238,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             const bool act = jj < per;
             const unsigned cr = act ? sh.off[rr + 1] - sh.off[rr] : 0u;
             const unsigned obase = act ? sh.off[rr] : 0u;
-            const size_t rbase = bufo + (size_t)rr * kFitPerBlock;
+            const size_t rbase = (size_t)rr * kFitPerBlock;
             uint32_t hw[kHold];
             float hz[kHold], ht[kHold];
 #pragma unroll
@@ -1230,9 +1248,9 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                 hz[u] = 0.0f;
                 ht[u] = 0.0f;
                 if (slot < cr) {
-                    hw[u] = ws.c_key[rbase + slot];
-                    hz[u] = ws.c_z[rbase + slot];
-                    ht[u] = ws.c_t[rbase + slot];
+                    hw[u] = c_key[rbase + slot];
+                    hz[u] = c_z[rbase + slot];
+                    ht[u] = c_t[rbase + slot];
                 }
             }
 #pragma unroll
@@ -1245,7 +1263,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
 #pragma unroll
                 for (int u = 0; u < kHold; ++u) {
                     const unsigned slot = s0 + (unsigned)(u * per);
-                    w[u] = slot < cr ? ws.c_key[rbase + slot] : 0u;
+                    w[u] = slot < cr ? c_key[rbase + slot] : 0u;
                 }
 #pragma unroll
                 for (int u = 0; u < kHold; ++u) {
@@ -1336,8 +1354,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
                     const unsigned slot = s0 + (unsigned)(u * per);
                     const uint32_t w = slot < cr ? sh.cand[obase + slot] : 0u;
                     use[u] = (w >> 31) && (w & 0x7fffffffu) <= thr;
-                    cz[u] = use[u] ? ws.c_z[rbase + slot] : 0.0f;
-                    ct[u] = use[u] ? ws.c_t[rbase + slot] : 0.0f;
+                    cz[u] = use[u] ? c_z[rbase + slot] : 0.0f;
+                    ct[u] = use[u] ? c_t[rbase + slot] : 0.0f;
                 }
 #pragma unroll
                 for (int u = 0; u < kHold; ++u) {
@@ -1582,13 +1600,18 @@ static int fit_blocks(int64_t N) {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Bytes before the exchanged elements: the header, the barrier flags, the partial sums, the histograms.
+static size_t fit_exchange_offset(int iters) {
+    const size_t hist = (size_t)(iters > 0 ? iters : 1) * kFitHistSlots * kFitHistWords * sizeof(unsigned);
+    return kFitHeader + align256(kFitMaxBlocks * 64) + align256(2 * kFitMaxBlocks * 5 * sizeof(uint64_t)) +
+           align256(hist);
+}
+
 size_t fit_workspace_bytes(int64_t N, int iters) {
     const int64_t n = N > 0 ? N : 1;
     const size_t nb = (size_t)fit_blocks(n);
-    const size_t hist = (size_t)(iters > 0 ? iters : 1) * kFitHistSlots * kFitHistWords * sizeof(unsigned);
-    const size_t cand = 2 * nb * (size_t)kFitThreads * fit_ept(n) * sizeof(uint32_t);
-    return kFitHeader + align256(kFitMaxBlocks * 64) + align256(2 * kFitMaxBlocks * 5 * sizeof(uint64_t)) +
-           align256(hist) + 3 * align256(cand);
+    const size_t cand = 6 * nb * (size_t)kFitThreads * fit_ept(n) * sizeof(uint32_t);
+    return fit_exchange_offset(iters) + cand;
 }
 
 // Polls of one barrier wait before it expires (~0.1 s at the default); lowered only by the test hook
@@ -1635,11 +1658,7 @@ int launch_fit(const FitLaunch& f, hipStream_t s) {
     ws.partials = (uint64_t*)p;
     p += align256(2 * kFitMaxBlocks * 5 * sizeof(uint64_t));
     ws.hist = (unsigned*)p;
-    p += align256((size_t)(f.iters > 0 ? f.iters : 1) * kFitHistSlots * kFitHistWords * sizeof(unsigned));
-    const size_t cand = align256(2 * (size_t)nb * kFitThreads * ept * sizeof(uint32_t));
-    ws.c_key = (uint32_t*)p;
-    ws.c_z = (float*)(p + cand);
-    ws.c_t = (float*)(p + 2 * cand);
+    ws.exch = (uint32_t*)((uint8_t*)f.workspace + fit_exchange_offset(f.iters));
     for (int b = 0; b < f.B; ++b) {
         FitArgs a{f.mode, f.z, f.tg, f.mask, f.logz, f.stride, f.lidar, f.conf, f.H, f.W, f.dh, f.dw,
                   f.N, f.iters, (float)(1.0 - (double)f.trim), f.min_points, b, f.st, f.info,
@@ -1848,6 +1867,20 @@ unsigned pmg_debug_fit_plan(unsigned mode) {
     const unsigned prev = (unsigned)g_fit_plan_debug;
     g_fit_plan_debug = mode <= 3 ? (int)mode : 0;
     return prev;
+}
+
+int pmg_debug_fit_exchange(int64_t N, int iters, int parity, int64_t* out) {
+    PMG_REQUIRE(out && N > 0 && N <= (int64_t)kFitMaxBlocks * kFitPerBlockMax, "bad size");
+    const int64_t per = (int64_t)kFitThreads * fit_ept(N), nb = fit_blocks(N);
+    const FitExchange ex = fit_exchange(nb * per, parity & 1);
+    const int64_t base = (int64_t)fit_exchange_offset(iters);
+    out[0] = nb;
+    out[1] = per;
+    out[2] = base + 4 * ex.key;
+    out[3] = base + 4 * ex.z;
+    out[4] = base + 4 * ex.t;
+    out[5] = base + 4 * ex.pairs;
+    return PMG_OK;
 }
 
 size_t pmg_fit_final_workspace_bytes(int B, int dh, int dw, int iters) {

@@ -182,6 +182,31 @@ def test_fit_plan_hook_round_trips(libpmg):
     assert libpmg.pmg_debug_fit_plan(0) == 0
 
 
+@pytest.mark.parametrize("N", [1, 4_096, 4_097, 9_000, 75 * 4_096, 1 << 19, (1 << 19) + 1, 762_048, 256 * 256 * 24,
+                               256 * 256 * 24 + 1, 1 << 21])
+def test_fit_exchange_regions_of_consecutive_stages_are_disjoint(libpmg, N):
+    """A block of the metric fit may write what stage n + 1 exchanges while a slower one still reads stage n's (either may be
+    a bracket stage: keys, z and targets, or a local stage: pairs): the two parities' regions share no byte, a stage's
+    own regions neither, and all lie in the workspace. (One block to 256, all three element layouts.)"""
+    for iters in (0, 4, 10):
+        total = libpmg.pmg_fit_workspace_bytes(N, iters)
+        regions = []
+        for parity in (0, 1):
+            out = (C.c_int64 * 6)()
+            assert libpmg.pmg_debug_fit_exchange(N, iters, parity, out) == 0
+            nb, per, key, z, t, pairs = out
+            assert nb * per >= N > (nb - 1) * per
+            span = lambda at, size: [(at + b * per * size, at + (b + 1) * per * size) for b in range(nb)]
+            bracket, local = span(key, 4) + span(z, 4) + span(t, 4), span(pairs, 8)
+            for own in (bracket, local):
+                own = sorted(own)
+                assert all(a[1] <= b[0] for a, b in zip(own, own[1:]))
+                assert own[0][0] >= 4096 and own[-1][1] <= total and own[0][0] % 16 == 0
+            regions.append(bracket + local)
+        hits = [(a, b) for a in regions[0] for b in regions[1] if a[0] < b[1] and b[0] < a[1]]
+        assert not hits, (len(hits), hits[:3])
+
+
 def test_fit_spin_limit_hook_round_trips(libpmg):
     prev = libpmg.pmg_debug_fit_spin_limit(7)
     assert prev == 1 << 23
