@@ -279,9 +279,10 @@ int pmg_fit_scale_shift_static(const float* z, const float* target, const uint8_
 unsigned pmg_debug_fit_spin_limit(unsigned polls);
 /* Test hook (no counterpart in the reference): makes the metric fit's round plans wrong on purpose, for the fits
  * enqueued after the call, so that tests reach the selection's fallbacks -- 1: each predicted bracket moved just
- * above its range (a window on the side that holds the k-th follows its miss); 2: each plan a window above every
- * finite residual (the radix passes follow its miss); 3: windows of 2^21-key bins (split passes); 0 (or any other
- * value) restores the normal plan. Results do not depend on the plan. Returns the previous mode. ABI version 5. */
+ * above its range (a window on the side that holds the k-th follows its miss), local rounds planned for a 64th of
+ * the moves (the state leaves their range after one); 2: each plan a window above every
+ * finite residual (the radix passes follow its miss); 3: windows of 2^21-key bins (split passes); 4: local rounds
+ * planned for states beside the current one (none may run); 0 (or any other value) restores the normal plan. Results do not depend on the plan. Returns the previous mode. ABI version 5. */
 unsigned pmg_debug_fit_plan(unsigned mode);
 /* Test hook (no counterpart in the reference; no GPU needed): where a fit of N elements keeps the elements that its blocks
  * exchange in a selection stage of the given parity. out[0] = blocks, out[1] = elements per block; byte offsets in the

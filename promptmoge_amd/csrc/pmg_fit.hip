@@ -669,6 +669,12 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         box.Dt = c * wt1 + wt0;
         return true;
     };
+    // Whether the current (s, t) lies in the box (1e-4 of it is kept for the margins' own rounding): what a classification
+    // over the box says of the current residuals holds only then. plan_box puts it there; its fp32 rounding may not.
+    auto in_box = [&]() -> bool {
+        const double du_now = ((double)s * zc + t) - ((double)box.s * zc + box.t);
+        return fabs((double)s - box.s) <= 0.9999 * box.Ds && fabs(du_now) <= 0.9999 * box.Du;
+    };
     bool use_local = false;  // the next round runs locally (box); the plan above is then its fallback
     auto plan_next = [&]() {
         // ---- the next round's plan. The threshold's move from round to round (in keys, which order like the
@@ -735,14 +741,20 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             dens_r = dens * (float)(f2u(fthr + h) - thr) * __builtin_amdgcn_rcpf(h);
             use_local = plan_box(have_prev, 7000.0f, 1.2f, 2.5f);
             if (a.plan_debug == 1) {
+                box.s = s;
+                box.t = t;
                 box.Ds *= 0.015625f;
                 box.Du *= 0.015625f;
+            } else if (a.plan_debug == 4) {
+                box.s += 3.0f * box.Ds;
             }
         }
         // Test hook: plans that are wrong on purpose, to exercise the fallbacks (the results must not change).
-        // 1: local rounds' boxes of a 64th of the moves (the next state leaves them), and a bracket just above its predicted range (the k-th usually lies below: a window on that side follows);
+        // 1: local rounds' boxes of a 64th of the moves around the current state (the next one leaves them), and a bracket
+        // just above its predicted range (the k-th usually lies below: a window on that side follows);
         // 2: every plan a window above +inf (it misses: the radix passes follow); 3: windows of 2^21-key bins from
-        // 2^24 keys below the threshold (split passes with a counted below-window part).
+        // 2^24 keys below the threshold (split passes with a counted below-window part); 4: local rounds' boxes beside the
+        // current state (no local round may run).
         if (a.plan_debug == 1 && plan_mode == 0) {
             const uint32_t w = hi - lo;
             lo = hi < 0xffffffffu ? hi + 1u : hi;
@@ -772,8 +784,9 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
     // block barrier each (0.45 us), sums, the solve: 4-5 us at 1000 elements, 7 at 6000, against a bracket round's 11 at
     // 75 blocks and 15 at 124 (publish, barrier, candidate loads). A fit of ten rounds on noisy maps, before and after:
     // 192x256 122 -> 74 us, 240x320 122 -> 89, 480x640 141 -> 98..121, 756x1008 206 -> 138..152.
-    // Runs rounds it0, it0 + 1, ... and returns how many were completed.
+    // Runs rounds it0, it0 + 1, ... and returns how many were completed: none where the current state is not in the box.
     auto run_local = [&](const int it0) -> int {
+        if (!in_box()) return 0;
         const unsigned kk = (unsigned)sh.kk;
         const int lane = tid & 63, wv = tid >> 6;
         int done = 0;
@@ -1056,7 +1069,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
             const double us = (double)s * zc + t;
             if (same || it0 + done >= a.iters || !(s >= s_lo && s <= s_hi && us >= u_lo && us <= u_hi)) return done;
             // ---- narrow where it drops most of more than 1600 elements and two rounds are left to gain by it
-            if (u <= 1600u || it0 + done + 2 > a.iters || !plan_box(true, fmax_(0.4f * (float)u, kLocalLow), 1.2f, 16.0f))
+            if (u <= 1600u || it0 + done + 2 > a.iters ||
+                !plan_box(true, fmax_(0.4f * (float)u, kLocalLow), 1.2f, 16.0f) || !in_box())
                 continue;
             double c5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
             uint32_t keep = 0;
@@ -1865,7 +1879,7 @@ unsigned pmg_debug_fit_spin_limit(unsigned polls) {
 
 unsigned pmg_debug_fit_plan(unsigned mode) {
     const unsigned prev = (unsigned)g_fit_plan_debug;
-    g_fit_plan_debug = mode <= 3 ? (int)mode : 0;
+    g_fit_plan_debug = mode <= 4 ? (int)mode : 0;
     return prev;
 }
 

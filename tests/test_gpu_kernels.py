@@ -791,6 +791,31 @@ def test_fit_local_rounds(gpu, libpmg, N):
     assert not 4_000 < N < 1_000_000 or 3 in codes[0], codes[0]
 
 
+@pytest.mark.parametrize("N", [4_095, 60_000, 300_000, 700_000])
+def test_fit_local_rounds_start_in_their_box(gpu, libpmg, N):
+    """Local rounds classify the elements for a box of states; planned for a box that the current state is not in (plan 4)
+    they do not run, and (s, t) and the threshold are the grid's own bit for bit."""
+    announce(f"fit local rounds planned beside the state N={N}")
+    rng = np.random.default_rng(N)
+    z = rng.uniform(0.4, 6, size=N).astype(np.float32)
+    t = (1.3 * z + 0.05 + 0.02 * z * rng.normal(size=N)).astype(np.float32)
+    t = np.where(rng.random(N) < 0.05, t * rng.uniform(0.4, 1.8, size=N), t).astype(np.float32)
+    m = rng.random(N) < 0.8
+    out = {}
+    try:
+        for mode in (0, 3, 4):
+            libpmg.pmg_debug_fit_plan(mode)
+            s_, t_, info = ops.fit_scale_shift(_t(z[None], gpu), _t(t[None], gpu), _t(m[None], gpu), iters=10, return_info=True)
+            torch.cuda.synchronize()
+            codes = {c for c, _ in _fit_trace(ops._fit_workspace(0, s_.device))}
+            assert int(info[0, 4]) == 0
+            assert (3 in codes) == (mode == 0), (mode, codes)
+            out[mode] = (float(s_[0]), float(t_[0]), int(info[0, 3]))
+    finally:
+        libpmg.pmg_debug_fit_plan(0)
+    assert out[4] == out[0] == out[3], out
+
+
 @pytest.mark.parametrize("name", ["B", "A", "H"])
 def test_fit_prompt_scene(gpu, name):
     announce(f"fit prompt scene={name}")
