@@ -289,6 +289,10 @@ unsigned pmg_debug_fit_plan(unsigned mode);
  * workspace of out[2] keys, out[3] z, out[4] targets (4 bytes an element, block after block) and out[5] pairs of z and
  * target (8 bytes an element). */
 int pmg_debug_fit_exchange(int64_t N, int iters, int parity, int64_t* out);
+/* Test hook (no counterpart in the reference; no GPU needed, host arrays): how the fit's local rounds class n elements over
+ * the box of states |s' - s| <= Ds, |u' - u| <= Du, |thr' - thr| <= Dt, u = s zc + t, box = {s, t, thr, zc, Ds, Du, Dt}:
+ * side[i] = -1 residual at or below the threshold in all of them, 1 above it in all, 0 unknown. */
+int pmg_debug_fit_class(const float* box, const float* z, const float* target, int64_t n, int8_t* side);
 int pmg_fit_scale_shift(const float* z, const float* target, const uint8_t* mask, int B, int64_t N, int iters,
                         float trim, int min_points, float* st, int32_t* info, void* workspace,
                         size_t workspace_bytes, void* stream);

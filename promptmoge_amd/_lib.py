@@ -122,6 +122,7 @@ SIGNATURES = {
     "pmg_debug_fit_spin_limit": (C.c_uint, [C.c_uint]),
     "pmg_debug_fit_plan": (C.c_uint, [C.c_uint]),
     "pmg_debug_fit_exchange": (i32, [i64, i32, i32, C.POINTER(i64)]),
+    "pmg_debug_fit_class": (i32, [vp, vp, vp, i64, vp]),
     "pmg_fit_scale_shift_static": (i32, [vp, vp, vp, i32, i64, i32, f32, i32, vp, vp, vp]),
     "pmg_fit_scale_shift": (i32, [vp, vp, vp, i32, i64, i32, f32, i32, vp, vp, vp, sz, vp]),
     "pmg_fit_prompt": (i32, [vp, i64, vp, vp, i32, i32, i32, i32, i32, i32, f32, i32, vp, vp, vp, sz, vp]),

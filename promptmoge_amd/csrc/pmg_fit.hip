@@ -294,20 +294,25 @@ __device__ inline void find_bin(FitShared& sh, unsigned rank, Load load, LoadBas
 // the mean z, which moves far less than t does), |thr' - thr| <= Dt.
 struct FitBox {
     float s, t, thr, zc, Ds, Du, Dt;
+    float sm, tm;  // the largest |s'| and |t'| of its states (fit_box_bounds)
 };
+__host__ __device__ inline void fit_box_bounds(FitBox& q) {
+    q.sm = __builtin_fabsf(q.s) + q.Ds;
+    q.tm = __builtin_fabsf(q.t) + q.Ds * __builtin_fabsf(q.zc) + q.Du;
+}
 // Whether an element's residual is below the threshold in every state of the box (`below` all ones), or above it
 // (`above` all ones), or may be either (both 0; also for NaN). |s' z + t' - tg| moves by at most Ds |z - zc| + Du, the
 // threshold by Dt; the residual's fp32 evaluation, here and in every later round, is off by at most
-// 2^-24 (3 |s z| + 2 |t| + |tg|) before the division and 2^-24 relative after it, and 2e-6 of the magnitudes covers both
-// evaluations four times over. The two tests are sign bits, not conditions: a condition combined with another goes
+// 2^-24 (3 |s' z| + 2 |t'| + |tg|) before the division and 2^-24 relative after it, and 2e-6 of the magnitudes covers both
+// evaluations four times over -- the magnitudes at the box's far end: few elements allow boxes of many times |s|, whose
+// states round far more coarsely than the middle one (with the middle's magnitudes, boxes of 1000 |s| misplaced elements). The two tests are sign bits, not conditions: a condition combined with another goes
 // through the scalar unit, and each such hop stalls a lone wave for ~25 cycles (measured: a ballot and its count 28
 // cycles, a vector operation 5), which made these per-element loops three times longer.
-__device__ inline void fit_class(const FitBox& q, float z, float tg, int& below, int& above) {
-    const float sz = q.s * z;
-    const float e = (sz + q.t) - tg;
+__host__ __device__ inline void fit_class(const FitBox& q, float z, float tg, int& below, int& above) {
+    const float e = (q.s * z + q.t) - tg;
     const float dm = __builtin_fmaxf(tg, 1e-3f);
     const float m = q.Ds * __builtin_fabsf(z - q.zc) + q.Du + q.Dt * dm +
-                    (2e-6f * (__builtin_fabsf(sz) + __builtin_fabsf(q.t) + __builtin_fabsf(tg)) + 1e-30f);
+                    (2e-6f * (q.sm * __builtin_fabsf(z) + q.tm + __builtin_fabsf(tg)) + 1e-30f);
     const float x = __builtin_fabsf(e) - q.thr * dm;
     below = (int)f2u(__builtin_fminf(x + m, 1e30f)) >> 31;  // (the minimum of a NaN and 1e30 is 1e30)
     above = (int)f2u(__builtin_fminf(m - x, 1e30f)) >> 31;
@@ -667,7 +672,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         box.Ds = c * ws1 + 1e-6f * __builtin_fabsf(s);
         box.Du = c * wu1 + 1e-6f * (__builtin_fabsf(s * zc) + __builtin_fabsf(t));
         box.Dt = c * wt1 + wt0;
-        return true;
+        fit_box_bounds(box);
+        return box.tm < 1e12f && box.thr + box.Dt < 1e15f;  // (below run_local's padding elements at every state)
     };
     // Whether the current (s, t) lies in the box (1e-4 of it is kept for the margins' own rounding): what a classification
     // over the box says of the current residuals holds only then. plan_box puts it there; its fp32 rounding may not.
@@ -787,6 +793,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
     // Runs rounds it0, it0 + 1, ... and returns how many were completed: none where the current state is not in the box.
     auto run_local = [&](const int it0) -> int {
         if (!in_box()) return 0;
+        fit_box_bounds(box);  // (a test hook may have moved the box)
         const unsigned kk = (unsigned)sh.kk;
         const int lane = tid & 63, wv = tid >> 6;
         int done = 0;
@@ -1894,6 +1901,18 @@ int pmg_debug_fit_exchange(int64_t N, int iters, int parity, int64_t* out) {
     out[3] = base + 4 * ex.z;
     out[4] = base + 4 * ex.t;
     out[5] = base + 4 * ex.pairs;
+    return PMG_OK;
+}
+
+int pmg_debug_fit_class(const float* box, const float* z, const float* target, int64_t n, int8_t* side) {
+    PMG_REQUIRE(box && z && target && side && n >= 0, "bad arguments");
+    FitBox q{box[0], box[1], box[2], box[3], box[4], box[5], box[6], 0.0f, 0.0f};
+    fit_box_bounds(q);
+    for (int64_t i = 0; i < n; ++i) {
+        int below, above;
+        fit_class(q, z[i], target[i], below, above);
+        side[i] = (int8_t)(above ? 1 : below);
+    }
     return PMG_OK;
 }
 

@@ -207,6 +207,42 @@ def test_fit_exchange_regions_of_consecutive_stages_are_disjoint(libpmg, N):
         assert not hits, (len(hits), hits[:3])
 
 
+@pytest.mark.parametrize("reach", [1e-5, 1e-2, 1.0, 30.0, 1e3, 1e5])
+def test_fit_classes_hold_over_the_whole_box(libpmg, reach):
+    """An element that the metric fit's local rounds class as below or above the threshold over a box of states is so in the
+    kernel's own fp32 residual at every state of it: boxes of `reach` times |s|, states near their ends, elements
+    around the mean z (where a box is widest in s for its uncertain elements), most with a residual within rounding of the
+    threshold there."""
+    F = np.float32
+    rng = np.random.default_rng(int(1e6 * reach))
+    n, bad, sure = 2_000, 0, 0
+    for _ in range(12):
+        zc, s, t, thr = F(rng.uniform(0.5, 5)), F(rng.uniform(0.2, 2)), F(rng.uniform(-1, 1)), F(10 ** rng.uniform(-6, -1))
+        Ds, Du = F(reach * s), F(rng.choice([1e-7, 1e-5, 1e-3]) * abs(s * zc + t))
+        Dt = F(thr * rng.choice([1e-3, 1e-2, 0.1]))
+        box = np.array([s, t, thr, zc, Ds, Du, Dt], F)
+        z = (zc * (1 + rng.choice([0, 1e-7, 1e-6, 1e-5, 1e-4, 1e-2], size=n) * rng.normal(size=n))).astype(F)
+        u0 = float(s) * float(zc) + float(t)
+        for k in range(200):
+            s2 = F(s + rng.choice([-1, 1]) * rng.uniform(0.3, 0.9998) * Ds)
+            t2 = F(u0 + (1 if k & 1 else -1) * 0.999 * Du - float(s2) * float(zc))
+            thr2 = F(thr + (1 if k & 2 else -1) * 0.999 * Dt)
+            if abs(float(s2) - s) > 0.9999 * Ds or abs(float(s2) * float(zc) + float(t2) - u0) > 0.9999 * Du:
+                continue
+            line = float(s2) * z.astype(np.float64) + float(t2)
+            fuzz = 2e-7 * rng.normal(size=n) * (abs(float(s2)) * z + abs(float(t2))) * rng.uniform(0, 1, n)
+            tg = (line / (1 + rng.choice([-1, 1], size=n) * float(thr2)) + fuzz).astype(F)
+            tg[::10] = 2 * line[::10]  # (a residual of a half)
+            side = np.empty(n, np.int8)
+            ptr = lambda a: a.ctypes.data_as(C.c_void_p)
+            assert libpmg.pmg_debug_fit_class(ptr(box), ptr(z), ptr(tg), n, ptr(side)) == 0
+            r = np.abs((s2 * z + t2) - tg) / np.maximum(tg, F(1e-3))
+            bad += int(((side < 0) & (r > thr2)).sum() + ((side > 0) & (r <= thr2)).sum())
+            sure += int((side != 0).sum())
+    assert bad == 0
+    assert reach > 0.1 or sure > 10_000, sure  # (the classes are of use where boxes are of the moves' size)
+
+
 def test_fit_spin_limit_hook_round_trips(libpmg):
     prev = libpmg.pmg_debug_fit_spin_limit(7)
     assert prev == 1 << 23
