@@ -338,7 +338,8 @@ __device__ inline float fit_rcp(float d) {
 // rounded, q faithful, r = e - q d by fused multiply-add, then RN(q + r y) = RN(e / d)). The compiler's own division
 // sequence is bit-identical, but passes a scale flag through VCC, so the N divisions ran one after the other: 16 elements
 // took 1.9 us of a round, 1.5 us this way with their masks. Operands outside the theorem's range (under- or overflow, all-ones divisors)
-// take the plain division, one branch for all N.
+// take the plain division, one branch for all N. Keys are below 2^31 (a NaN's sign is dropped): the loops compare them as
+// signed numbers, and a NaN orders above every number.
 template <int N>
 __device__ inline void fit_keys(float s, float t, const float* z, const float* tg, const float* rc, bool odd_targets,
                                 uint32_t* key) {
@@ -363,7 +364,7 @@ __device__ inline void fit_keys(float s, float t, const float* z, const float* t
             float e = s * z[j];
             e = e + t;
             e = e - tg[j];
-            key[j] = f2u(__builtin_fabsf(e) / fmax_(tg[j], 1e-3f));
+            key[j] = f2u(__builtin_fabsf(e) / fmax_(tg[j], 1e-3f)) & 0x7fffffffu;  // (inf / inf is -NaN)
         }
     }
 }

@@ -816,6 +816,27 @@ def test_fit_local_rounds_start_in_their_box(gpu, libpmg, N):
     assert out[4] == out[0] == out[3], out
 
 
+@pytest.mark.parametrize("N", [40, 3_000, 50_000, 300_000, 800_000])
+@pytest.mark.parametrize("n_inf", [1, 4])
+def test_fit_infinite_targets(gpu, N, n_inf):
+    """Infinite targets inside the mask on a constant z: the first solve's t is infinite, every finite target's residual too,
+    and the infinite targets' is no number (inf - inf, then inf / inf), which sorts last and is never kept: from the second
+    round on the fit is that of the finite targets, as in the oracle."""
+    announce(f"fit infinite targets N={N} n={n_inf}")
+    rng = np.random.default_rng(N)
+    z = np.full(N, 2, np.float32)
+    t = (3 + 0.1 * rng.normal(size=N)).astype(np.float32)
+    m = rng.random(N) < 0.8
+    m[:36] = True
+    t[5:5 + 9 * n_inf:9][:n_inf] = np.inf
+    for iters in (2, 4, 10):
+        with np.errstate(all="ignore"):
+            so, to = ofit.fit_f64(z[None], t[None], m[None], iters=iters)
+        s_, t_ = ops.fit_scale_shift(_t(z[None], gpu), _t(t[None], gpu), _t(m[None], gpu), iters=iters)
+        assert np.isfinite(to[0])
+        _close_st(float(s_[0]), float(t_[0]), so[0], to[0])
+
+
 @pytest.mark.parametrize("name", ["B", "A", "H"])
 def test_fit_prompt_scene(gpu, name):
     announce(f"fit prompt scene={name}")
