@@ -346,9 +346,13 @@ __host__ __device__ inline int xcd_group(int64_t nunits) { return nunits >= 8 * 
 
 // Blocks of a host-sized launch that walks nchunk chunks with at most `most` blocks: each XCD has a block for every
 // chunk that it is dealt, as far as they go. (A grid of nchunk blocks gave the later XCDs fewer blocks than chunks: int8
-// C = 128, 22 chunks of 512 rows: 101 us, whole rounds of 8 blocks 52; 157 chunks in groups: 104 and 55.)
-static int64_t walk_blocks(int64_t nchunk, int64_t most) {
-    const int64_t n = xcd_group(nchunk) ? most : (nchunk + 7) / 8 * 8;
+// C = 128, 22 chunks of 512 rows: 101 us, whole rounds of 8 blocks 52; 157 chunks in groups: 104 and 55.) Staged launches in
+// slices of output channels keep contiguous bands at any size: every slice deals its chunks to the same XCDs, so that the
+// groups' remainder would weigh once per slice (16-bit C = 512, 157 chunks in 8 slices: two groups on two XCDs, one on
+// the other six; groups / bands, us, by rows: 17.5k 640 / 485, 20k 766 / 487, 38k 1141 / 957, 100k 2547 / 2389; C = 256:
+// 42k 306 / 233, 70k 448 / 385, 130k 615 / 619).
+static int64_t walk_blocks(int64_t nchunk, int64_t most, bool bands = false) {
+    const int64_t n = !bands && xcd_group(nchunk) ? most : (nchunk + 7) / 8 * 8;
     return n < most ? n : most;
 }
 
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(kG2Threads, 1) void spconv_g2_k(ConvArgs a) {
         for (int kk = 0; kk < WPP; ++kk) dst[(wv + kG2Waves * (part * WPP + kk)) * 64 + lane] = st[kk];
     };
 
-    const int gi = kDev ? 0 : xcd_group(nunit);
+    const int gi = kDev || NS != C ? 0 : xcd_group(nunit);  // (slices: bands, see walk_blocks)
     for (int kq = bi;; kq += nbx) {
         const int un = gi ? ((kq / gi) * nx + x) * gi + kq % gi : c0 + kq;
         if (un >= (gi ? nunit : c1)) break;
@@ -1244,7 +1248,7 @@ static int launch_g2f(const ConvArgs& a, int epilogue, hipStream_t s) {
     constexpr int T = RB <= 128 ? 4 : (RB <= 512 ? 2 : 1), CHUNK = kG2Waves * T * 16;
     constexpr int PFV = RB >= 512 ? 4 : 1;  // weight operands read ahead (measured: 3 % faster at C = 256 / 512)
     const int64_t nchunk = (a.M + CHUNK - 1) / CHUNK;
-    const dim3 grid((unsigned)(walk_blocks(nchunk, cus)), (unsigned)(C / (16 * NB))), blk(kG2Threads);
+    const dim3 grid((unsigned)(walk_blocks(nchunk, cus, C / (16 * NB) > 1)), (unsigned)(C / (16 * NB))), blk(kG2Threads);
     switch (epilogue) {
         case PMG_EPI_ACC: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_ACC, NB, T, PFV, 2, false, E>), grid, blk, 0, s, a); break;
         case PMG_EPI_BIAS: hipLaunchKernelGGL((spconv_g2_k<C, PMG_EPI_BIAS, NB, T, PFV, 2, false, E>), grid, blk, 0, s, a); break;

@@ -450,7 +450,8 @@ def test_conv_f32(gpu, Ci, Co):
 
 _FLOAT_CASES = [("f16", 32, m) for m in (1, 127, 98_303, 98_305, 614_401)] + [("bf16", 48, 129), ("f16", 48, 5_001)] + \
     [("bf16", 64, m) for m in (2, 1_025, 73_728, 73_729, 131_073)] + [("f16", 96, 3_000), ("bf16", 96, 17)] + \
-    [("f16", 128, m) for m in (15, 8_192, 8_193, 16_384, 16_385)] + [("bf16", 128, 8_200), ("f16", 256, 1), ("f16", 256, 65), ("bf16", 256, 8_192), ("f16", 256, 8_193)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
+    [("f16", 128, m) for m in (15, 8_192, 8_193, 16_384, 16_385)] + [("bf16", 128, 8_200), ("f16", 256, 1), ("f16", 256, 65), ("bf16", 256, 8_192), ("f16", 256, 8_193),
+     ("f16", 256, 33_025), ("bf16", 512, 16_257)] + [("f32", c, m) for c, m in ((16, 1_000), (16, 1), (32, 129), (48, 257),
                                                                                  (48, 3_001), (64, 16), (64, 5_000))]
 
 
