@@ -117,11 +117,14 @@ def test_gauge_three_frames_degree3_odd_grid(gpu):
 
 
 @pytest.mark.parametrize("case,hw", [("exact", (120, 160)), ("wide", (61, 83)), ("half_ties", (97, 131)), ("one_block", (16, 16)),
-                                     ("many", (300, 470))])
+                                     ("many", (300, 470)), ("exact", (733, 719)), ("wide", (301, 517)), ("wide", (733, 719)),
+                                     ("half_ties", (301, 517)), ("half_ties", (733, 719)), ("many", (1201, 1003))])
 def test_gauge_median_paths(gpu, case, hw):
     """The median's ways: all residuals below the histogram's range and more of them than a block's list holds ("exact":
     a constant gauge), above it ("wide": a log-gauge noise of about 1), most of one value ("half_ties"), a frame of one
-    block, and one of 256 blocks whose medians' bins hold several hundred."""
+    block, and one of 256 blocks whose medians' bins hold several hundred; bins of more than a block's list in each way, on
+    frames below and above 2^19 pixels (the values counted by every block, or by a launch of their own), odd
+    sizes (the second frame's list is not a multiple of 16 bytes away)."""
     announce(f"gauge median paths: {case} {hw}")
     h, w = hw
     rng = np.random.default_rng(h)
