@@ -24,8 +24,9 @@
 // power-of-two width, LDS histogram per block, merged by atomics), and the stage runs on the bin that holds the
 // k-th; a bracket that misses is followed by such a window on the side that holds the k-th; round 0 (no threshold yet)
 // takes a window over residuals 2^-15 .. 2, and round 1, where the first trim may have dropped the threshold by octaves, a
-// window over 16 octaves around round 0's threshold. A window that misses is followed by radix passes over the whole key range (bins of 2^21 keys, then 2^10 within the first bin, then single keys, each
-// only while the bin holds more than 2048 keys); when one key value holds the k-th and more than kCandCap
+// window over 16 octaves around round 0's threshold (unless the trim moved little: plan_next). A window that misses is
+// followed by radix passes over the whole key range (bins of 2^21 keys, then 2^10 within the first bin, then single
+// keys, each only while the bin holds more than 2048 keys); when one key value holds the k-th and more than kCandCap
 // elements, it is the threshold and the sums take one more barrier.
 // The stage checks that its bracket holds the k-th, so a prediction can cost time but never change a result.
 // Once the moves are small, the remaining rounds need no device-wide barrier at all: each block runs them by itself on the
@@ -51,7 +52,7 @@ namespace pmg {
 
 constexpr int kFitThreads = 256;
 constexpr int kFitWaves = kFitThreads / 64;
-constexpr int kFitEPTMax = 32;                         // elements per thread, in registers (16 or 32)
+constexpr int kFitEPTMax = 32;                         // elements per thread, in registers (16, 24 or 32)
 constexpr int kFitPerBlockMax = kFitThreads * kFitEPTMax;  // 8192
 constexpr int kFitMaxBlocks = kFitThreads;             // N <= 2^21
 constexpr int kFitBins = 2048;
@@ -651,8 +652,8 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         mv_t = fmax_(fmax_(__builtin_fabsf(dt), 0.5f * mv_t), 1e-4f * fthr);
     };
     // The box for the rounds ahead. The moves keep their direction while they are large and shrink to a jitter, so the
-    // box reaches 0.8 c times the last move along it, and 0.3 c times the decayed magnitudes to either side; the first
-    // trim moves the threshold by -0.6 to +1.3 % (seen), mostly under 0.5: +-0.8 % after round 0. c as large as
+    // box reaches 0.8 c times the last move along it, and 0.3 c times the decayed magnitudes to either side; after round 0,
+    // which has no move of the threshold to go by, +-0.8 % of it (only where plan_next expects it to stay within). c as large as
     // `target` uncertain elements allow, in [cmin, cmax] (above cmax while they are under kLocalLow: a wide box costs nothing
     // there); false if that is not to be had (or nothing finite can be said).
     auto plan_box = [&](bool have, float target, float cmin, float cmax) -> bool {
@@ -698,11 +699,17 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         if (sh.total_cand >= 64u || dens <= 0.0f)
             dens = (float)sh.total_cand * __builtin_amdgcn_rcpf((float)(sh.bhi_last - sh.blo_last) + 1.0f);
         plan_mode = 2;
-        if (!have_prev && sh.total_cand >= 64u && dens * 0.016f * (float)((thr & 0x7fffffu) | 0x800000u) < 4000.0f &&
-            box_width(mv_s, mv_u, 0.0f) < 0.25f * u2f(thr)) {
-            // after round 0 of a noisy map (the first trim moved the residuals by less than a quarter of the threshold):
-            // a bracket of +-0.8 % usually holds the threshold (13 us at 480x640 against 20 by the window); the window below
-            // on a miss
+        // After round 0: whether the first trim leaves the threshold within 0.8 %, from the mean move of the residuals that it
+        // caused. Seen (fits of synthetic rooms, 96x128 to 480x640): moves of up to 0.12 thresholds and under 0.016 go with
+        // threshold moves of 0 to 0.8 % (5 mm noise) and 0.6 % (half the targets outliers), larger ones with 2.6 to 3.5 %
+        // (20 % noise), 12 to 14 % (a bent map) and 33 % (unrelated targets); maps that one refiner step made: -1.5 % (A, passes
+        // and misses), -2.4 % (T) and +10 % (H, both refused). A local series that fails at once costs 6 to 10 us, a missed
+        // bracket 5: 192x256, four rounds, 20 % noise 92 us, unrelated targets 74; refused 75 and 62.
+        const float first = box_width(mv_s, mv_u, 0.0f);
+        const bool steady = have_prev || (first < 0.125f * u2f(thr) && first < 0.016f);
+        if (!have_prev && steady && sh.total_cand >= 64u &&
+            dens * 0.016f * (float)((thr & 0x7fffffu) | 0x800000u) < 4000.0f) {
+            // a bracket of +-0.8 % (13 us at 480x640 against 20 by the window; 24 where it misses and the window follows)
             plan_mode = 0;
             lo = f2u(0.992f * u2f(thr));
             hi = f2u(1.008f * u2f(thr));
@@ -748,7 +755,7 @@ __global__ __launch_bounds__(kFitThreads) void fit_k(FitArgs a) {
         if (local_fails < 2) {
             const float fthr = u2f(thr), h = fthr * 9.765625e-4f;
             dens_r = dens * (float)(f2u(fthr + h) - thr) * __builtin_amdgcn_rcpf(h);
-            use_local = plan_box(have_prev, 7000.0f, 1.2f, 2.5f);
+            use_local = steady && plan_box(have_prev, 7000.0f, 1.2f, 2.5f);
             if (a.plan_debug == 1) {
                 box.s = s;
                 box.t = t;
