@@ -910,7 +910,8 @@ __global__ __launch_bounds__(64 * NWV, 1) void spconv_g2r_k(ConvArgs a) {
 //   fp16 C = 256      75 / 56 / 42      78 / 108 / 62      298 / 312 / 184   -
 //   fp16 C = 512     102 / 107 / 90    289 / 309 / 199     -                 -
 //   int8 C = 128      52 / 19 / 19      52 / 19 / 19       54 / 47 / 41      109 / 162 / -
-//   int8 C = 256     103 / 39 / 33     186 / 71 / 50      599 / 180 / 115    -        (one wave per 16 rows for staged)
+//   int8 C = 256     103 / 39 / 33     186 / 71 / 50      599 / 180 / 115   1880 / 595 / -  (one wave per 16 rows for staged;
+//                    400k rows 3.9 ms / 1.25, 1M 9.1 / 2.9)
 // Tiles of 128 rows, waves of 128 x 32 or 64 x 64, and blocks of 8 waves were slower (C = 256, 11k rows, fragment order:
 // 62 - 90 us): they leave one block to a CU, or fewer waves than the loads' latency asks for.
 //
